@@ -231,3 +231,64 @@ def test_unet_adam_steps_reduce_loss(require_gpu):
     net = UNet(c, seed=3)
     losses = [net.train_step(x, t, lr=1e-3) for _ in range(30)]
     assert losses[-1] < 0.5 * losses[0], losses[::5]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,H,W,Cin,Cout,relu,shift", [
+    (1, 1, 1, 32, 32, 1, 0),        # one pixel: all but the centre tap outside
+    (3, 15, 31, 32, 32, 0, 0),      # one short of a tile in both directions, images joined inside a fragment
+    (2, 16, 30, 64, 96, 1, 0),      # whole rows of tiles, images meeting at a fragment's end; 32-channel tiles
+    (2, 17, 33, 96, 64, 0, 0),      # one past a tile in both directions
+    (70, 3, 2, 32, 64, 1, 0),       # images much narrower than a fragment
+    (1, 20, 37, 32, 32, 1, 1),      # arrays off the 16-byte alignment
+])
+def test_conv3x3_bf16_tile_edges(require_gpu, N, H, W, Cin, Cout, relu, shift):
+    import torch
+    from mbrec import _lib
+    print(f"conv3x3 edges N={N} H={H} W={W} Cin={Cin} Cout={Cout}", flush=True)
+    g = rng(100 + H)
+    x = _bf16_tensor(g.standard_normal((N, H, W, Cin)))
+    w = _bf16_tensor(g.standard_normal((Cout, 3, 3, Cin)) / np.sqrt(9 * Cin))
+    b = torch.as_tensor(g.standard_normal(Cout).astype(np.float32))
+
+    def place(t):
+        buf = torch.zeros(t.numel() + shift, dtype=t.dtype, device="cuda")
+        buf[shift:] = t.reshape(-1).cuda()
+        return buf[shift:]
+    xd, wd, bd = place(x), place(w), b.cuda()
+    yd = place(torch.full((N, H, W, Cout), 7.0, dtype=torch.bfloat16))
+    _lib.check(_lib.lib().mbrec_conv3x3_bf16(xd.data_ptr(), wd.data_ptr(), bd.data_ptr() if relu else None,
+                                             yd.data_ptr(), N, H, W, Cin, Cout, relu, _lib.stream_handle()))
+    want = torch.nn.functional.conv2d(x.double().permute(0, 3, 1, 2), w.double().permute(0, 3, 1, 2), padding=1)
+    if relu:
+        want = torch.relu(want + b.double().view(1, -1, 1, 1))
+    want = want.permute(0, 2, 3, 1).numpy()
+    got = yd.float().cpu().numpy().reshape(want.shape)
+    # outputs rounded to bfloat16 (2^-9 relative), FP32 sums of 9 Cin products below that
+    assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c,N,H,W", [(32, 3, 24, 40), (32, 1, 8, 8), (64, 2, 40, 24)])
+def test_unet_ragged_grids_match_oracle(require_gpu, c, N, H, W):
+    """Grids whose levels end inside tiles (level 4 odd, down to one pixel), both base widths."""
+    from mbrec.warmstart import UNet
+    print(f"unet ragged c={c} N={N} H={H} W={W}", flush=True)
+    g = rng(31)
+    th = U.he_init(c, 32).astype(np.float32).astype(np.float64)
+    x = g.uniform(0.0, 1.0, (N, H, W)).astype(np.float32)
+    t = (0.5 * x + 0.1 * g.uniform(0, 1, (N, H, W))).astype(np.float32)
+    net = UNet(c)
+    net.set_params(th)
+    want, _ = U.forward(th, x.astype(np.float64), c, quant=True)
+    # the oracle's own distance to 64 bits here is 0.3 % (c = 32) and 1.3 % (c = 64); flipped roundings stay below it
+    assert rel_l2(net.forward(x).cpu().numpy(), want) < 2e-2
+    loss, grad = net.gradients(x, t)
+    lw, gw, _ = U.loss_and_grad(th, x.astype(np.float64), t.astype(np.float64), c, quant=True)
+    assert abs(loss - lw) < 2e-3 * lw
+    lay, _ = U.layout(c)
+    for (ci, co, k, wo, bo), name in zip(lay, U.LAYER_NAMES):
+        # a flipped bfloat16 rounding or ReLU mask of one pixel moves a deep layer's gradient by up
+        # to 2-3 % at these sizes (any order of the FP32 sums); a wrong tap, tile edge or
+        # channel by far more
+        assert rel_l2(grad[wo:bo + co], gw[wo:bo + co]) < 8e-2, name
