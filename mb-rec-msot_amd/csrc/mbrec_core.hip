@@ -57,7 +57,7 @@ static void free_work(Plan *p)
         if (q) (void)hipFree(q);
     p->d_bins = p->d_hpart = p->d_imgI = p->d_img_tmp = p->d_sino_tmp = p->d_gpart = p->d_sband = nullptr;
     p->d_img_slot = nullptr;
-    p->sband_nwave = p->sband_nfb = 0;
+    p->sband_nrun = p->sband_nfb = p->sband_rb = 0;
     p->bcap = 0;
     p->work_bytes = 0;
 }
@@ -90,16 +90,18 @@ int ensure_work(Plan *p, int B)
         free_work(p);
         return rc;
     }
-    // band-form SIR forward rows (batches): waves of nfb = TS + 1 - maxlen first samples each
-    if (B > 1 && p->use_sir && p->d_srec && p->sir_maxlen <= kSirBandTS) {
-        const int nfb = kSirBandTS + 1 - std::max(p->sir_maxlen, 1);
-        const int nwave = (p->sp_n + nfb - 1) / nfb;
-        if ((rc = dalloc(&p->d_sband, (size_t)p->D * nwave * (3 * kSirBandTS + 1) * Bp, &acc))) {
+    // band-form SIR forward rows: a band's taps and the sample after them stay within 32 samples
+    if (p->use_sir && p->d_srec && p->sir_maxlen < kSirBandTS) {
+        const int nfb = p->sir_maxlen <= kSirBandTS - kSirBandShift ? kSirBandShift : kSirBandTS - p->sir_maxlen;
+        const int rb = nfb == kSirBandShift ? kSirBandRun : 1;
+        const int nrun = (p->sp_n + nfb * rb - 1) / (nfb * rb);
+        if ((rc = dalloc(&p->d_sband, (size_t)p->D * nrun * sband_rows(rb) * 3 * Bp, &acc))) {
             free_work(p);
             return rc;
         }
-        p->sband_nwave = nwave;
+        p->sband_nrun = nrun;
         p->sband_nfb = nfb;
+        p->sband_rb = rb;
     }
     // the two zero rows after the last detector's bins (pairs outside the bin range read them)
     MBREC_HIP(hipMemset(p->d_bins + (size_t)p->D * p->geom.NB * Bp, 0, sizeof(float) * 2 * Bp));
@@ -338,10 +340,10 @@ static int build_sir_pull(Plan *p, const std::vector<int32_t> &slot_pix, const s
     p->d_sirw = nullptr;
     p->sp_lo = 0;
     p->sp_n = 0;
-    if ((size_t)p->Nsir_build * stride >= ((size_t)1 << 31) || maxlen >= (1 << 15) || p->P >= (1 << 28) ||
+    if ((size_t)p->Nsir_build * stride + 64 >= ((size_t)1 << 31) || maxlen >= (1 << 15) || p->P >= (1 << 28) ||
         span >= (1 << 15))
         return MBREC_OK;   // the packed record does not fit: the SIR forward keeps the bucketed form only
-    std::vector<float> sw((size_t)p->Nsir_build * stride, 0.0f);
+    std::vector<float> sw((size_t)p->Nsir_build * stride + 64, 0.0f);
     for (int k = 0; k < p->Nsir_build; ++k)
         for (int i = 0; i < win[2 * (size_t)k + 1]; ++i)
             sw[(size_t)k * stride + kSirWinPad + i] = sirf[(size_t)k * Ls + win[2 * (size_t)k] + i];
@@ -396,6 +398,7 @@ static int build_sir_pull(Plan *p, const std::vector<int32_t> &slot_pix, const s
         (rc = upload(p->d_srec_off, off.data(), off.size())) || (rc = upload(p->d_sirw, sw.data(), sw.size())))
         return rc;
     p->table_bytes += p->srec_bytes;
+    p->sirw_zero = p->Nsir_build * stride;
     p->sp_lo = lo;
     p->sp_n = n_nf;
     return MBREC_OK;

@@ -38,7 +38,11 @@ struct HatTaps {
 constexpr int kTileRowsMax = 256;   // tile gathers: longest bin window they stage (rows)
 constexpr int kRecPad = 512;   // zero records after the pull table (runs of up to 512 read past the end)
 constexpr int kSirWinPad = 32;   // zero weights on each side of a window in the pull form's SIR table
-constexpr int kSirBandTS = 30;   // samples per wave of the band-form SIR forward
+constexpr int kSirBandTS = 32;   // samples per wave of the band-form SIR forward
+// bands per run of the band-form SIR forward: eight where the accumulators can move up by eight
+// samples between bands (windows of at most 24 taps), else one; rows a run leaves per bin phase
+constexpr int kSirBandShift = 8, kSirBandRun = 4;
+static inline int sband_rows(int rb) { return rb > 1 ? kSirBandShift * rb + 24 : kSirBandTS; }
 
 struct BinGeom {
     float phi1, phi2;            // sorted interior breakpoint phases in [0,1)
@@ -153,8 +157,9 @@ struct Plan {
     float *d_sino_tmp = nullptr; // [B][D][nT]       samples before/after the IR filter
     float *d_gpart = nullptr;    // [max(8 B, 16)][P]  partial images of the detector-grouped gathers
     float *d_img_slot = nullptr; // [Pd]  one sinogram's image in slot order (pull forward)
-    float *d_sband = nullptr;    // [D][band waves][3 kSirBandTS + 1][Bp]  band-form SIR forward rows (B > 1)
-    int sband_nwave = 0, sband_nfb = 0;
+    float *d_sband = nullptr;    // [D][runs][rows][3][Bp]  band-form SIR forward rows
+    int sband_nrun = 0, sband_nfb = 0, sband_rb = 0;
+    int sirw_zero = 0;           // first of 64 zeros at the end of d_sirw
     size_t table_bytes = 0;
     size_t work_bytes = 0;
     int pins = 0;                // batches whose captured graphs use this plan's buffers

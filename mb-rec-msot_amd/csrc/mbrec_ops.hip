@@ -1854,104 +1854,270 @@ __global__ __launch_bounds__(256) void k_fwd_sir_pull_bl(const int4 *__restrict_
     }
 }
 
-// SIR forward for batches, band form, pass 1 (lane = sinogram): wave w takes the records
-// whose first affected sample nf lies in its band [a, a + nfb), a = lo + w nfb, so every
-// record is visited once; its taps land on samples a .. a + TS - 1 (TS >= nfb - 1 + maxlen)
-// and the wave keeps their 3 TS + 1 bins in registers.  A record's TS weights from sample
-// a on come from the zero-margin weights table (offset nf - a before its first tap).  The
-// bin of sample -1's phase-2 u-part and the phase-0 part at sample span are dropped
-// where they fall in the wave's range (the reference's range check).  The wave's rows go
-// to its slot of the band scratch; pass 2 adds the overlapping slots.
-template <int TS>
-__device__ __forceinline__ void sir_band_phase(float (&acc)[3 * TS + 1], const int4 *__restrict__ rec, int rs,
-                                               int re, const float *__restrict__ imgI,
-                                               const float *__restrict__ sirw, int a, int Bp, int bo, int m)
+// SIR forward for batches, band form, pass 1 (FP32 matrix cores): out[sample][sinogram] =
+// sum over records of weight[sample][record] x pixel[record][sinogram], a contraction over
+// records whose weight matrix has the records' windows as columns.  A wave takes a run of rb
+// bands of nfb first samples; the records of a band [a, a + nfb) have their taps (and the
+// u-part of phase 2, one sample on) on the 32 samples from a.  Two records per product
+// 32x32x2: A = 32 weights of each from the zero-margin table (one 128-byte run per record)
+// times 1 - u or u, B = the records' pixel rows (32 sinograms).  Every record is visited once,
+// for 32 NC sinograms at a time; the accumulators are the samples' three bins.
+// With nfb = 8 (windows of at most 24 taps) the next band's samples are the same accumulators
+// eight rows on -- four registers of the 32x32 layout -- so a band's first eight samples
+// leave for the band scratch and the rest moves up (registers only); a run ends with 24 rows
+// that the next run adds to (rb = 1: all 32 rows leave, any nfb <= 32 - longest window).
+// Taps on samples outside [0, span) have their weights masked (the reference's range check).
+// Pass 2 adds the overlapping rows in run order.
+// Bound by the matrix cores: 2 products of 64 cycles per two records and 32 sinograms (at
+// 400^2 and 64 sinograms 2.1 ms of matrix time); without any loads the loop still takes 0.9 of
+// its 1.2 ms at 300^2 x 28 (0.6 ms of matrix time).  Forward operator against the vector form
+// that issued 60 FMAs per record and 64 lanes: 300^2 x 28 4.98 -> 1.49 ms, 400^2 x 64
+// 8.88 -> 4.02 ms, 300^2 x 2 4.86 -> 1.3 ms.  Four bands per run: the scratch is 1.75 rows per
+// sample, and one wave per workgroup keeps the last waves short (eight bands: 0.2 ms more).
+// 64 sinograms per wave read each weight once for both halves (two waves of 32: 8 % more).
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr int kSirRunTail = 24;   // rows of a run (rb > 1) past its own first samples
+
+template <int NC, int M>
+__device__ __forceinline__ void sir_mf_phase(f32x16 (&acc)[3][NC], const int4 *__restrict__ rec, int rs, int re,
+                                             const float *__restrict__ imgI, const float *__restrict__ sirw, int a,
+                                             int span, int zoff, int Bp, const int (&col)[NC])
 {
-    for (int r = rs; r < re; ++r) {
-        const int4 e = rec[r];
-        const float c = imgI[(size_t)(e.x & 0x0fffffff) * Bp + bo];
-        const int t0 = ((e.y << 16) >> 16) - a;   // in [0, nfb)
-        const float *w = sirw + (size_t)e.w - t0;   // w[t]: weight of the tap on sample a + t
-        float h[TS];
-#pragma unroll
-        for (int t = 0; t < TS; ++t) h[t] = w[t];
+    constexpr int U = 8;   // products whose operands are in flight while the previous U run
+    const int lane = threadIdx.x & 63, t = lane & 31, hl = lane >> 5;
+    const bool in0 = a + t >= 0 && a + t < span, in1 = a + t >= 1 && a + t <= span;   // sample, sample before
+    int4 e = rec[max(min(rs + lane, re - 1), 0)];
+    for (int c0 = rs; c0 < re; c0 += 64) {
+        // lane = record; past the end: the last record with zero weights
+        const int px = e.x & 0x0fffffff, wo = c0 + lane < re ? e.w - (((e.y << 16) >> 16) - a) : zoff;
         const float u = __int_as_float(e.z);
-        const float c0 = c * (1.0f - u), c1 = c * u;
+        const int nk = min(32, (re - c0 + 1) / 2);
+        e = rec[max(min(c0 + 64 + lane, re - 1), 0)];   // the next 64, in flight during these
+        float A0[2][U], A1[2][U], uu[2][U], Bv[2][U][NC];
+        auto load = [&](int k, int s) __attribute__((always_inline)) {
 #pragma unroll
-        for (int t = 0; t < TS; ++t) {
-            acc[3 * t + m] += c0 * h[t];
-            acc[3 * t + m + 1] += c1 * h[t];
+            for (int q = 0; q < U; ++q) {
+                const int src = min(2 * (k + q) + hl, 63);
+                const float *w = sirw + __shfl(wo, src) + t;
+                A0[s][q] = w[0];
+                A1[s][q] = M == 2 ? w[-1] : 0.0f;
+                uu[s][q] = __shfl(u, src);
+                const float *row = imgI + (size_t)__shfl(px, src) * Bp;
+#pragma unroll
+                for (int n = 0; n < NC; ++n) Bv[s][q][n] = row[col[n]];
+            }
+        };
+        auto mul = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < U; ++q) {
+                const float w0 = in0 ? A0[s][q] : 0.0f, w1 = M == 2 ? (in1 ? A1[s][q] : 0.0f) : w0;
+                const float f0 = w0 * (1.0f - uu[s][q]), f1 = w1 * uu[s][q];
+#pragma unroll
+                for (int n = 0; n < NC; ++n)
+                    acc[M][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(f0, Bv[s][q][n], acc[M][n], 0, 0, 0);
+#pragma unroll
+                for (int n = 0; n < NC; ++n)
+                    acc[(M + 1) % 3][n] =
+                        __builtin_amdgcn_mfma_f32_32x32x2f32(f1, Bv[s][q][n], acc[(M + 1) % 3][n], 0, 0, 0);
+            }
+        };
+        load(0, 0);
+        for (int k = 0; k < nk; k += 2 * U) {   // records past nk are the last one with zero weights
+            // (the barriers keep the loads ahead of the products, which the scheduler would issue first)
+            load(k + U, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            mul(0);
+            if (k + U >= nk) break;
+            __builtin_amdgcn_sched_barrier(0);
+            if (k + 2 * U < nk) load(k + 2 * U, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            mul(1);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
 }
 
-template <int TS>
-__global__ __launch_bounds__(256) void k_fwd_sir_band(const int4 *__restrict__ rec, const int32_t *__restrict__ off,
+template <int NC>
+__global__ __launch_bounds__(64) void k_fwd_sir_band(const int4 *__restrict__ rec, const int32_t *__restrict__ off,
                                                       const float *__restrict__ imgI, const float *__restrict__ sirw,
-                                                      float *__restrict__ scratch, int span, int lo, int n_nf,
-                                                      int nfb, int nwave, int Bp)
+                                                      float *__restrict__ scratch, int D, int span, int lo, int n_nf,
+                                                      int nfb, int rb, int nrun, int zoff, int Bp)
+{
+    const int lane = threadIdx.x & 63, j = lane & 31;
+    const int run = blockIdx.x / D, d = blockIdx.x - run * D;
+    const int b0 = blockIdx.y * 32 * NC;
+    int a = lo + run * nfb * rb, col[NC];
+#pragma unroll
+    for (int n = 0; n < NC; ++n) col[n] = min(b0 + 32 * n + j, Bp - 1);
+    const int rows = rb > 1 ? 8 * rb + kSirRunTail : 32;
+    float *dst = scratch + ((size_t)d * nrun + run) * rows * 3 * Bp + b0 + j + (size_t)(4 * (lane >> 5)) * 3 * Bp;
+    f32x16 acc[3][NC];
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+        for (int n = 0; n < NC; ++n)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[m][n][i] = 0.0f;
+    // rows 8 g + 4 (lane / 32) + i of the accumulators (register 4 g + i) to row r0 + ...
+    auto store = [&](int g, int r0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+#pragma unroll
+                for (int n = 0; n < NC; ++n)
+                    if (b0 + 32 * n + j < Bp) dst[((size_t)(r0 + i) * 3 + m) * Bp + 32 * n] = acc[m][n][4 * g + i];
+    };
+    const int32_t *o = off + (size_t)d * 3 * (n_nf + 1);
+    for (int band = 0; band < rb; ++band, a += nfb) {
+        if (band) {
+            store(0, 8 * (band - 1));
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+#pragma unroll
+                for (int n = 0; n < NC; ++n)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[m][n][i] = i < 12 ? acc[m][n][(i + 4) & 15] : 0.0f;
+        }
+        const int ia = a - lo, ib = min(ia + nfb, n_nf);
+        if (ia >= n_nf) continue;
+        sir_mf_phase<NC, 0>(acc, rec, o[ia], o[ib], imgI, sirw, a, span, zoff, Bp, col);
+        sir_mf_phase<NC, 1>(acc, rec, o[n_nf + 1 + ia], o[n_nf + 1 + ib], imgI, sirw, a, span, zoff, Bp, col);
+        sir_mf_phase<NC, 2>(acc, rec, o[2 * (n_nf + 1) + ia], o[2 * (n_nf + 1) + ib], imgI, sirw, a, span, zoff, Bp, col);
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) store(g, 8 * (rb - 1) + 8 * g);
+}
+
+// SIR forward for one sinogram, band form, pass 1: the same runs and bands on the vector ALUs.
+// Lane = four samples (of 32) x one of eight records: a record's 32 weights are eight 16-byte
+// loads of consecutive lanes (4-byte aligned: a window starts anywhere).  64 records are read
+// at once (lane = record, with its pixel value split into the 1 - u and u parts) and handed
+// out eight at a time, three cross-lane reads per eight records: with one sample per lane and
+// two records at a time those reads cost a tenth more (0.81 ms at 400^2 against 0.78 ms per forward; the
+// lane-group form k_fwd_sir_pull1, which reads a scattered weight per lane and visits every
+// record from two waves, 1.88 ms and remains for windows of more than 31 taps).  The samples
+// a lane group holds rotate by two between bands instead of moving.  The blocks of an XCD work on
+// the same few distances and share the windows in its L2.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// t0: first of this lane's samples, from a
+template <int M>
+__device__ __forceinline__ void sir_band1_phase(float (&acc)[3][4], const int4 *__restrict__ rec, int rs, int re,
+                                                const float *__restrict__ img, const float *__restrict__ sirw, int a,
+                                                int t0, int span, int zoff)
+{
+    constexpr int U = 4;   // groups of eight records whose weights are in flight together
+    const int lane = threadIdx.x & 63, g = lane >> 3;
+    float s0[4] = {0.0f, 0.0f, 0.0f, 0.0f}, s1[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (rs >= re) return;
+    int4 e = rec[min(rs + lane, re - 1)];
+    float c = img[e.x & 0x0fffffff];
+    for (int c0 = rs; c0 < re; c0 += 64) {
+        // past the end: the last record with zero weights
+        const int wo = c0 + lane < re ? e.w - (((e.y << 16) >> 16) - a) : zoff;
+        const float u = __int_as_float(e.z), ca = c * (1.0f - u), cb = c * u;
+        const int nk = min(8, (re - c0 + 7) / 8);
+        const bool more = c0 + 64 < re;
+        if (more) e = rec[min(c0 + 64 + lane, re - 1)];
+        for (int k = 0; k < nk; k += U) {
+            f32x4u A[U];
+#pragma unroll
+            for (int q = 0; q < U; ++q)
+                A[q] = *reinterpret_cast<const f32x4u *>(sirw + __shfl(wo, 8 * (k + q) + g) + t0);
+            if (more && k == 0) c = img[e.x & 0x0fffffff];
+#pragma unroll
+            for (int q = 0; q < U; ++q) {
+                const float va = __shfl(ca, 8 * (k + q) + g), vb = __shfl(cb, 8 * (k + q) + g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s0[i] = fmaf(A[q][i], va, s0[i]);
+                    s1[i] = fmaf(A[q][i], vb, s1[i]);
+                }
+            }
+        }
+    }
+    // taps on samples outside [0, span) are dropped; the u-part of phase 2 is the next sample's
+    // phase 0 (no tap on the last of the 32 samples)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (a + t0 + i < 0 || a + t0 + i >= span) s0[i] = s1[i] = 0.0f;
+    const float before = M == 2 ? __shfl(s1[3], (lane & 56) | ((lane - 1) & 7)) : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        acc[M][i] += s0[i];
+        acc[(M + 1) % 3][i] += M == 2 ? (i ? s1[i ? i - 1 : 0] : before) : s1[i];
+    }
+}
+
+__global__ __launch_bounds__(256) void k_fwd_sir_band1(const int4 *__restrict__ rec, const int32_t *__restrict__ off,
+                                                       const float *__restrict__ img, const float *__restrict__ sirw,
+                                                       float *__restrict__ scratch, int D, int span, int lo, int n_nf,
+                                                       int nfb, int rb, int nrun, int zoff)
 {
     const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-    if (w >= nwave) return;   // no barriers in this kernel
-    const int d = blockIdx.y;
-    const int b = blockIdx.z * 64 + lane;
-    const int bo = min(b, Bp - 1);
-    const int a = lo + w * nfb;
-    const int ia = w * nfb, ib = min(ia + nfb, n_nf);
-    float acc[3 * TS + 1];
+    const int nd = (D + 3) / 4, k = blockIdx.x >> 3, run = (k / nd) * 8 + (blockIdx.x & 7);   // as k_fwd_sir_band
+    const int d = __builtin_amdgcn_readfirstlane((k % nd) * 4 + (threadIdx.x >> 6));
+    if (d >= D || run >= nrun) return;   // no barriers in this kernel
+    int a = lo + run * nfb * rb;
+    const int rows = rb > 1 ? 8 * rb + kSirRunTail : 32;
+    float *dst = scratch + ((size_t)d * nrun + run) * rows * 3;
+    float acc[3][4];
 #pragma unroll
-    for (int k = 0; k < 3 * TS + 1; ++k) acc[k] = 0.0f;
+    for (int i = 0; i < 12; ++i) acc[i / 4][i % 4] = 0.0f;
     const int32_t *o = off + (size_t)d * 3 * (n_nf + 1);
-    // phase 2 first: the u-part of sample -1 (row 0) is dropped before other phases add there
-    sir_band_phase<TS>(acc, rec, o[2 * (n_nf + 1) + ia], o[2 * (n_nf + 1) + ib], imgI, sirw, a, Bp, bo, 2);
+    for (int band = 0; band < rb; ++band, a += nfb) {
+        const int t0 = 4 * ((lane - 2 * band) & 7);   // eight samples on per band: two lanes down
+        const int ia = a - lo, ib = min(ia + nfb, n_nf);
+        if (ia < n_nf) {
+            sir_band1_phase<0>(acc, rec, o[ia], o[ib], img, sirw, a, t0, span, zoff);
+            sir_band1_phase<1>(acc, rec, o[n_nf + 1 + ia], o[n_nf + 1 + ib], img, sirw, a, t0, span, zoff);
+            sir_band1_phase<2>(acc, rec, o[2 * (n_nf + 1) + ia], o[2 * (n_nf + 1) + ib], img, sirw, a, t0, span, zoff);
+        }
+        // the first eight samples leave (all 32 after the last band): sums over the eight record groups
+        const bool leave = t0 < 8 || band + 1 == rb;
 #pragma unroll
-    for (int t = 0; t < TS; ++t)
-        if (a + t == -1) acc[3 * t + 3] = 0.0f;
-    // phase 0: the part at sample span (row 3 span) is dropped, the u-part of span - 1 kept
-    float keep = 0.0f;
+        for (int m = 0; m < 3; ++m)
 #pragma unroll
-    for (int t = 0; t < TS; ++t)
-        if (a + t == span) keep = acc[3 * t];
-    sir_band_phase<TS>(acc, rec, o[ia], o[ib], imgI, sirw, a, Bp, bo, 0);
-#pragma unroll
-    for (int t = 0; t < TS; ++t)
-        if (a + t == span) acc[3 * t] = keep;
-    sir_band_phase<TS>(acc, rec, o[(n_nf + 1) + ia], o[(n_nf + 1) + ib], imgI, sirw, a, Bp, bo, 1);
-    if (b >= Bp) return;
-    float *dst = scratch + (((size_t)d * nwave + w) * (3 * TS + 1)) * Bp + b;
-#pragma unroll
-    for (int k = 0; k < 3 * TS + 1; ++k) dst[(size_t)k * Bp] = acc[k];
+            for (int i = 0; i < 4; ++i) {
+                float v = acc[m][i];
+                v += __shfl_xor(v, 8);
+                v += __shfl_xor(v, 16);
+                v += __shfl_xor(v, 32);
+                if (leave && lane < 8) dst[(8 * band + t0 + i) * 3 + m] = v;
+                if (leave) acc[m][i] = 0.0f;
+            }
+    }
 }
 
-// pass 2: bins[d][j][b] = sum over the waves whose rows [3 a_w, 3 (a_w + TS)] hold j, in
-// wave order (rows of samples outside [0, span] are never asked for)
-template <int TS>
+// pass 2: bins[d][j][b] = sum over the runs whose rows hold bin j, in run order (run r covers
+// samples lo + r step .. + rows - 1; rows of samples outside [0, span] are never asked for);
+// thread = V sinograms of a bin (V = 4 for batches, whose Bp is a multiple of 4)
+template <int V>
 __global__ __launch_bounds__(256) void k_fwd_sir_band_sum(const float *__restrict__ scratch,
-                                                          float *__restrict__ bins, int NB, int lo, int nfb,
-                                                          int nwave, int Bp)
+                                                          float *__restrict__ bins, int NB, int lo, int step, int rows,
+                                                          int nrun, int Bp)
 {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;   // (j, b) of detector blockIdx.y
-    if (i >= (size_t)NB * Bp) return;
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const int i = blockIdx.x * 256 + threadIdx.x, BV = Bp / V;   // (j, b / V) of detector blockIdx.y
+    if (i >= NB * BV) return;
     const int d = blockIdx.y;
-    const int j = (int)(i / Bp), b = (int)(i - (size_t)j * Bp);
-    // wave w covers rows 3 (lo + w nfb) .. 3 (lo + w nfb + TS)
-    const int wlo = max(0, (j - 3 * (lo + TS) + 3 * nfb - 1) / (3 * nfb)), whi = min(nwave - 1, (j - 3 * lo) / (3 * nfb));
-    // up to 8 rows in flight per step, added in wave order (absent rows add 0)
-    float acc = 0.0f;
-    for (int w0 = wlo; w0 <= whi; w0 += 8) {
-        float v[8];
+    const int j = i / BV, b = V * (i - j * BV), n = j / 3 - lo, m = j - 3 * (j / 3);
+    const int whi = min(nrun - 1, n / step), wlo = max(0, (n - rows + step) / step);
+    vec acc = (vec)(0.0f);
+    for (int w0 = wlo; w0 <= whi; w0 += 4) {   // up to 4 rows in flight, added in run order (absent rows add 0)
+        vec v[4];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int w = w0 + k, r = j - 3 * (lo + w * nfb);
-            v[k] = (w <= whi && r >= 0 && r <= 3 * TS)
-                       ? scratch[(((size_t)d * nwave + w) * (3 * TS + 1) + r) * Bp + b]
-                       : 0.0f;
+        for (int k = 0; k < 4; ++k) {
+            const int w = w0 + k, r = n - w * step;
+            v[k] = (vec)(0.0f);
+            if (w <= whi && r < rows)
+                v[k] = *reinterpret_cast<const vec *>(scratch + ((((size_t)d * nrun + w) * rows + r) * 3 + m) * Bp + b);
         }
 #pragma unroll
-        for (int k = 0; k < 8; ++k) acc += v[k];
+        for (int k = 0; k < 4; ++k) acc += v[k];
     }
-    bins[((size_t)d * NB + j) * Bp + b] = acc;
+    *reinterpret_cast<vec *>(bins + ((size_t)d * NB + j) * Bp + b) = acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -2925,8 +3091,8 @@ static void scatter_bl(Plan *p, const float *imgI, int B, int Bp, hipStream_t s)
 // scatter launch choice: > 0 record-lane kernel with that LDS batch chunk, < 0
 // batch-lane kernel with lane groups of -value sinograms
 // SIR forward in pull form (records of build_sir_pull): scatter choices of their own, the
-// bins written directly (no bucket windows).  kSirPull: for one sinogram the lane-group
-// kernel (the default there), else the batch-lane kernel with 24 samples and 2 records in
+// bins written directly (no bucket windows).  kSirPull: for one sinogram the band form on the
+// vector ALUs (windows of more than 31 taps: the lane-group kernel; the default there), else the batch-lane kernel with 24 samples and 2 records in
 // flight per wave; kSirPull + 1 .. 3: batch-lane kernels with (16 samples, 4 records),
 // (16, 2), (32, 1); kSirBand (batches; the default there): every record visited once by
 // the wave of its first-sample band, the overlapping wave rows summed in a second pass
@@ -2934,11 +3100,16 @@ constexpr int kSirPull = 1000, kSirPullVariants = 5, kSirBand = kSirPull + 4;
 
 static bool is_sir_pull(int c) { return c >= kSirPull && c < kSirPull + kSirPullVariants; }
 
+// tables and scratch of the band form are there (windows of at most 31 taps)
+static bool sir_band_ok(const Plan *p, int Bp)
+{
+    return p->use_sir && p->d_srec && p->d_sirw && p->d_sband && p->sband_nfb >= 1 && p->bcap >= 1 &&
+           batch_stride(p->bcap) >= Bp;
+}
+
 static bool sir_pull_ok(const Plan *p, int Bp, int c = kSirPull)
 {
-    if (c == kSirBand)
-        return p->use_sir && p->d_srec && p->d_sirw && Bp > 1 && p->d_sband && p->sband_nfb >= 1 &&
-               p->bcap >= 1 && batch_stride(p->bcap) >= Bp;
+    if (c == kSirBand) return Bp > 1 && sir_band_ok(p, Bp);
     return p->use_sir && p->d_srec && p->d_sirw && is_sir_pull(c) && (c == kSirPull || Bp > 1);
 }
 
@@ -3532,21 +3703,34 @@ static int launch_scatter(Plan *p, const float *imgI, int B, int Bp, hipStream_t
 {
     if (p->pull) return launch_pull(p, imgI, Bp, s);
     if (const int sc = scatter_choice(p, Bp); is_sir_pull(sc)) {
-        if (Bp == 1) {
-            const int span = p->geom.nT + 2 * p->geom.K;
+        const int span = p->geom.nT + 2 * p->geom.K;
+        if (sc == kSirBand || (Bp == 1 && sir_band_ok(p, Bp))) {
+            const int step = p->sband_nfb * p->sband_rb;
+            const int zoff = p->sirw_zero + 1;   // zeros from one before to 31 after
+            const unsigned nwg = (unsigned)((p->sband_nrun + 7) / 8 * 8 * ((p->D + 3) / 4));
+            // 64 sinograms per wave where a part of the second half is used, else 32
+            const auto launch = [&](auto kern, int nc) {
+                hipLaunchKernelGGL(kern, dim3(p->sband_nrun * p->D, (Bp + 32 * nc - 1) / (32 * nc)), dim3(64), 0, s,
+                                   p->d_srec, p->d_srec_off, imgI, p->d_sirw, p->d_sband, p->D, span, p->sp_lo, p->sp_n,
+                                   p->sband_nfb, p->sband_rb, p->sband_nrun, zoff, Bp);
+            };
+            const auto sum = [&](auto kern, int v) {
+                hipLaunchKernelGGL(kern, dim3((unsigned)(((size_t)p->geom.NB * Bp / v + 255) / 256), p->D), dim3(256), 0, s,
+                                   (const float *)p->d_sband, p->d_bins, p->geom.NB, p->sp_lo, step,
+                                   sband_rows(p->sband_rb), p->sband_nrun, Bp);
+            };
+            if (Bp == 1)
+                hipLaunchKernelGGL(k_fwd_sir_band1, dim3(nwg), dim3(256), 0, s, p->d_srec, p->d_srec_off, imgI,
+                                   p->d_sirw, p->d_sband, p->D, span, p->sp_lo, p->sp_n, p->sband_nfb, p->sband_rb,
+                                   p->sband_nrun, zoff);
+            else if (Bp > 32) launch(k_fwd_sir_band<2>, 2);
+            else launch(k_fwd_sir_band<1>, 1);
+            if (Bp == 1) sum(k_fwd_sir_band_sum<1>, 1);
+            else sum(k_fwd_sir_band_sum<4>, 4);
+        } else if (Bp == 1) {
             const int nblk = (span + 1 + 59) / 60;   // 4 waves x 15 samples per workgroup
             hipLaunchKernelGGL(k_fwd_sir_pull1, dim3(nblk, p->D), dim3(256), 0, s, p->d_srec, p->d_srec_off, imgI,
                                p->d_sirw, p->d_bins, p->geom.NB, span, p->sp_lo, p->sp_n, p->sir_maxlen);
-        } else if (sc == kSirBand) {
-            constexpr int TS = kSirBandTS;
-            const int span = p->geom.nT + 2 * p->geom.K;
-            hipLaunchKernelGGL((k_fwd_sir_band<TS>), dim3((p->sband_nwave + 3) / 4, p->D, (Bp + 63) / 64), dim3(256),
-                               0, s, p->d_srec, p->d_srec_off, imgI, p->d_sirw, p->d_sband, span, p->sp_lo, p->sp_n,
-                               p->sband_nfb, p->sband_nwave, Bp);
-            hipLaunchKernelGGL((k_fwd_sir_band_sum<TS>),
-                               dim3((unsigned)(((size_t)p->geom.NB * Bp + 255) / 256), p->D), dim3(256), 0, s,
-                               (const float *)p->d_sband, p->d_bins, p->geom.NB, p->sp_lo, p->sband_nfb,
-                               p->sband_nwave, Bp);
         } else if (sc == kSirPull + 1) sir_pull_bl<16, 4>(p, imgI, Bp, s);
         else if (sc == kSirPull + 2) sir_pull_bl<16, 2>(p, imgI, Bp, s);
         else if (sc == kSirPull + 3) sir_pull_bl<32, 1>(p, imgI, Bp, s);

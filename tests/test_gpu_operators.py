@@ -212,6 +212,37 @@ def test_every_launch_variant_matches_oracle(sir, B):
     plan.set_launch(B, -1, 0)
 
 
+@pytest.mark.parametrize("length,B", [(1, 1), (24, 1), (25, 1), (31, 1), (32, 1), (24, 2), (25, 33), (31, 32), (32, 4),
+                                      (8, 64), (24, 67)])
+def test_sir_forward_band_edges(length, B):
+    """The band forms of the SIR forward at the window lengths where they change (24: bands that
+    slide, 31: longest window of a band, 32: the forms without bands) and at the edges of a
+    wave's sinograms; random travel times put taps on both ends of the sample axis, every
+    record list is odd-sized or empty somewhere, and 67 detectors leave workgroups partly idle."""
+    import torch
+    from mbrec.model import DevicePlan
+    Nz, Nx, D, nT, R, Ls = 11, 13, 67, 150, 2.6666666666666665, 35
+    _log(f"sir band edges length={length} B={B}")
+    g = rng(500 + length)
+    tt = random_tt(Nz * Nx, D, nT, R, 7, margin=-6)
+    nsir = 9
+    sir = g.standard_normal((Ls, nsir))
+    se = np.zeros((2, nsir), dtype=np.int32)
+    for k in range(nsir):
+        n = length if k == 0 else int(g.integers(1, length + 1))
+        s0 = int(g.integers(1, Ls - n + 2))
+        se[:, k] = (s0, s0 + n - 1)
+    se[:, nsir - 1] = (3, 2)          # no taps
+    sidx = g.integers(1, nsir + 1, size=(Nz * Nx, D)).astype(np.int32)
+    plan = DevicePlan(Nz, Nx, D, nT, R, np.ascontiguousarray(tt.T),
+                      sir=(np.ascontiguousarray(sidx.T), np.ascontiguousarray(sir.T), np.ascontiguousarray(se.T)))
+    x = g.uniform(0, 1, (B, Nx, Nz))
+    yo = np.transpose(O.forward_sir(x.reshape(B, -1), sidx, tt, sir, nT, se, R), (0, 2, 1))
+    y = plan.forward(torch.tensor(x, dtype=torch.float32).cuda(), model=False).cpu().numpy()
+    assert rel_l2(y, yo) < TOL_OP
+    assert np.abs(y - yo).max() < 1e-4 * np.abs(yo).max()
+
+
 @pytest.mark.parametrize("sir", [False, True])
 @pytest.mark.parametrize("B", [1, 64])
 def test_autotuned_launch_matches_oracle(sir, B):
