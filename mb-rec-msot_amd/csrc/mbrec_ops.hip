@@ -18,6 +18,7 @@
 #include "mbrec_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mbrec {
 
@@ -2557,65 +2558,82 @@ __global__ __launch_bounds__(1024) void k_gather_tt(
 // read from the one being filled (and does not wait for the fill before reading).
 constexpr int kTaMaxD = 512;   // detectors whose window origins the async tile gather keeps in LDS
 
-template <int NCH>
+//
+// LB sinograms per workgroup (64, 32, 16): a wave's 16 pixels are then 16, 8 or 4 steps of
+// 64 / LB pixels, so that small batches keep their lanes busy and move LB columns of a window
+// only.  With LB <= 32 two workgroups share a CU (80 KB of LDS each), one waiting for its
+// detector's loads while the other interpolates.
+template <int NCH, int LB>
 struct TaLayout {
     static constexpr int ZR = 64 * NCH, RS = ZR + 2;    // window rows, then two zero rows
-    static constexpr int BUF = RS * 64 + 2 * 256;       // floats per buffer: rows, then 256 table entries
+    static constexpr int BUF = RS * LB + 2 * 256;       // floats per buffer: rows, then 256 table entries
 };
 
-template <int G, int NCH>
-__global__ __launch_bounds__(1024) void k_gather_ta(
+template <int G, int NCH, int LB>
+__global__ __launch_bounds__(1024, LB <= 32 ? 8 : 4) void k_gather_ta(
     const int2 *__restrict__ ttab, const int2 *__restrict__ twin, const int32_t *__restrict__ pix,
     const float *__restrict__ bins, float *__restrict__ out, int D, int NB, int P, int B, int Bp, float scale,
     int bins_bytes, int ttab_bytes, const int32_t *__restrict__ tord)
 {
-    using L = TaLayout<NCH>;
+    using L = TaLayout<NCH, LB>;
+    constexpr int RPL = 256 / LB;                          // rows one wave load moves
+    constexpr int NL = L::ZR / RPL, NF = NL / 16, NR = NL % 16;   // wave loads: NF by every wave, one more by NR waves
+    constexpr int NP = LB / 4;                             // pixels per lane (16 per wave)
     __shared__ __attribute__((aligned(16))) float s0[L::BUF], s1[L::BUF], s2[L::BUF];
-    __shared__ int2 tw[kTaMaxD];   // the tile's window origins
+    __shared__ int32_t tw[(kTaMaxD + G - 1) / G];   // the tile's window origins
     // tord: the tile of each workgroup (XCD-aware order; -1: a padding workgroup, which
     // exits before any barrier), or null: workgroup x = tile x
     const int tile = tord ? tord[blockIdx.x] : (int)blockIdx.x;
     if (tile < 0) return;
-    const int grp = blockIdx.y % G, b0 = (blockIdx.y / G) * 64;
+    const int grp = blockIdx.y % G, b0 = (blockIdx.y / G) * LB;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int DG = (D + G - 1) / G, dbeg = grp * DG, dend = min(D, dbeg + DG);
-    for (int i = threadIdx.x; i < 2 * 64; i += 1024) {   // the zero rows of the three buffers
-        s0[L::ZR * 64 + i] = 0.0f;
-        s1[L::ZR * 64 + i] = 0.0f;
-        s2[L::ZR * 64 + i] = 0.0f;
+    for (int i = threadIdx.x; i < 2 * LB; i += 1024) {   // the zero rows of the three buffers
+        s0[L::ZR * LB + i] = 0.0f;
+        s1[L::ZR * LB + i] = 0.0f;
+        s2[L::ZR * LB + i] = 0.0f;
     }
-    for (int i = threadIdx.x; i < D; i += 1024) tw[i] = twin[(size_t)tile * D + i];
+    for (int i = threadIdx.x; i < dend - dbeg; i += 1024) tw[i] = twin[(size_t)tile * D + dbeg + i].x;
     __syncthreads();
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(bins), (short)0, bins_bytes, kBufferWord3);
     const __amdgpu_buffer_rsrc_t rt =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<int2 *>(ttab), (short)0, ttab_bytes, kBufferWord3);
     const int rowb = 4 * Bp;
-    // load c of wave w moves rows 4 (16 c + w) .. + 3: lane l takes row + l / 16, columns b0 + 4 (l % 16) ..
-    const int vo = (lane >> 4) * rowb + 4 * (b0 + 4 * (lane & 15));
+    // load c of wave w moves rows RPL (16 c + w) ..: lane l takes row + l / (LB / 4), columns b0 + 4 (l % (LB / 4)) ..
+    const int vo = (lane / (LB / 4)) * rowb + 4 * (b0 + 4 * (lane % (LB / 4)));
     auto stage = [&](int d, float *bb) __attribute__((always_inline)) {
-        const int so = (d * NB + __builtin_amdgcn_readfirstlane(tw[d].x)) * rowb;
+        const int so = (d * NB + __builtin_amdgcn_readfirstlane(tw[d - dbeg])) * rowb;
 #pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            const int r0 = 4 * (16 * c + wv);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)(bb + r0 * 64),
-                                                     16, vo, so + r0 * rowb, 0, 0);
+        for (int c = 0; c < NF + (NR > 0); ++c) {
+            const int r0 = RPL * (16 * c + wv);
+            if (c < NF || wv < NR)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)(bb + r0 * LB),
+                                                         16, vo, so + r0 * rowb, 0, 0);
         }
         if (wv < 2)   // table entries 128 w .. 128 w + 127 of (tile, d): 16 bytes (2 entries) per lane
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rt, (__attribute__((address_space(3))) void *)(bb + L::RS * 64 + 256 * wv), 16, 16 * lane,
+                rt, (__attribute__((address_space(3))) void *)(bb + L::RS * LB + 256 * wv), 16, 16 * lane,
                 (int)((((size_t)tile * D + d) * 256 + 128 * wv) * sizeof(int2)), 0, 0);
     };
-    float acc[16], part[16];
+    // sums of eight detectors in FP32, added up in FP64 with LB <= 32 (as close to the exact sum as the
+    // compensated sums of the record- and batch-lane forms: 3.1e-7 against 3.0e-7 of the operator at
+    // 301 x 333 x 28).  64 registers at most there: 66 would leave one workgroup per CU (0.41 / 0.29 ms)
+    using Sum = std::conditional_t<(LB <= 32), double, float>;
+    Sum acc[NP];
+    float part[NP];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) acc[k] = part[k] = 0.0f;
+    for (int k = 0; k < NP; ++k) acc[k] = part[k] = 0.0f;
     // one detector: wait for its loads, barrier, start the fill two ahead, interpolate
     auto step = [&](int d, const float *rd, float *wr) __attribute__((always_inline)) {
         if (d + 1 < dend) {   // this wave's loads for d are done (those for d + 1 may be in flight)
+            static_assert(NR == 0 || NR >= 2, "the waves that move table entries are among the NR");
             if (wv < 2)
-                __builtin_amdgcn_s_waitcnt(kWaitVm(NCH + 1));
+                __builtin_amdgcn_s_waitcnt(kWaitVm(NF + (NR > 0) + 1));
+            else if (NR > 0 && wv < NR)
+                __builtin_amdgcn_s_waitcnt(kWaitVm(NF + 1));
             else
-                __builtin_amdgcn_s_waitcnt(kWaitVm(NCH));
+                __builtin_amdgcn_s_waitcnt(kWaitVm(NF));
         } else {
             __builtin_amdgcn_s_waitcnt(kWaitVm(0));
         }
@@ -2623,24 +2641,25 @@ __global__ __launch_bounds__(1024) void k_gather_ta(
         // barrier: a full fence here would also wait for the loads of d + 1)
         __builtin_amdgcn_s_barrier();
         if (d + 2 < dend) stage(d + 2, wr);
-        const int4 *te = reinterpret_cast<const int4 *>(rd + L::RS * 64) + 8 * wv;   // this wave's 16 entries
-        const float *wb = rd + lane;
-        float g0[16], g1[16], uu[16];
+        // this wave's 16 entries; lane group l / LB takes entries NP (l / LB) ..
+        const int4 *te = reinterpret_cast<const int4 *>(rd + L::RS * LB) + 8 * wv + (lane / LB) * (NP / 2);
+        const float *wb = rd + lane % LB;
+        float g0[NP], g1[NP], uu[NP];
 #pragma unroll
-        for (int k2 = 0; k2 < 8; ++k2) {
-            const int4 e = te[k2];   // entries 2 k2, 2 k2 + 1 (same address in every lane)
-            g0[2 * k2] = wb[e.x * 64];
-            g1[2 * k2] = wb[e.x * 64 + 64];
+        for (int k2 = 0; k2 < NP / 2; ++k2) {
+            const int4 e = te[k2];   // entries 2 k2, 2 k2 + 1 (same address in every lane of a group)
+            g0[2 * k2] = wb[e.x * LB];
+            g1[2 * k2] = wb[e.x * LB + LB];
             uu[2 * k2] = __int_as_float(e.y);
-            g0[2 * k2 + 1] = wb[e.z * 64];
-            g1[2 * k2 + 1] = wb[e.z * 64 + 64];
+            g0[2 * k2 + 1] = wb[e.z * LB];
+            g1[2 * k2 + 1] = wb[e.z * LB + LB];
             uu[2 * k2 + 1] = __int_as_float(e.w);
         }
 #pragma unroll
-        for (int k = 0; k < 16; ++k) part[k] += fmaf(uu[k], g1[k] - g0[k], g0[k]);
+        for (int k = 0; k < NP; ++k) part[k] += fmaf(uu[k], g1[k] - g0[k], g0[k]);
         if (((d - dbeg) & 7) == 7) {
 #pragma unroll
-            for (int k = 0; k < 16; ++k) {
+            for (int k = 0; k < NP; ++k) {
                 acc[k] += part[k];
                 part[k] = 0.0f;
             }
@@ -2661,12 +2680,12 @@ __global__ __launch_bounds__(1024) void k_gather_ta(
             if (d + 5 < dend) step(d + 5, s2, s1);
         }
     }
-    const int b = b0 + lane;
+    const int b = b0 + lane % LB;
     if (b >= B) return;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const float v = acc[k] + part[k];
-        const int px = pix[(size_t)tile * 256 + 16 * wv + k];
+    for (int k = 0; k < NP; ++k) {
+        const float v = (float)(acc[k] + part[k]);
+        const int px = pix[(size_t)tile * 256 + 16 * wv + (lane / LB) * NP + k];
         if (px < 0) continue;
         if (G > 1)
             out[((size_t)grp * B + b) * P + px] = v;
@@ -3148,11 +3167,14 @@ static bool pull_choice_ok(const Plan *p, int c, int Bp)
     return false;
 }
 
-static int default_pull_choice(int Bp)
+// wave-uniform forms (a wave's bins, lane = sinogram) from 12 sinograms on: with raw-buffer
+// image rows above 32, where the image rows fit 32-bit offsets.  Stage times against the former
+// choices (batch-lane groups of 16 and 32 below 64, one bin per thread at 12): 400^2 x 48
+// 0.79 / 3.38 ms, 301 x 333 x 28 0.51 / 1.49 ms, x 16 0.46 / 0.90 ms (x 8: 0.32 ms, kept).
+static int default_pull_choice(const Plan *p, int Bp)
 {
-    if (Bp >= 64) return -964;
-    if (Bp >= 32) return -32;
-    if (Bp >= 16) return -16;
+    if (Bp > 32 && pull_choice_ok(p, -964, Bp)) return -964;
+    if (Bp >= 12) return -864;
     if (Bp % 8 == 0) return 8;
     if (Bp % 4 == 0) return 4;
     return Bp == 1 ? 2 : 1;
@@ -3644,7 +3666,7 @@ static void fwd_pull_wt(Plan *p, const float *imgI, int Bp, hipStream_t s, int J
 static int launch_pull(Plan *p, const float *imgI, int Bp, hipStream_t s)
 {
     // one sinogram: the tile form over sorted rows (2 detectors per workgroup) when its tables exist
-    const int dflt = (Bp == 1 && pull_choice_ok(p, 11, Bp)) ? 11 : default_pull_choice(Bp);
+    const int dflt = (Bp == 1 && pull_choice_ok(p, 11, Bp)) ? 11 : default_pull_choice(p, Bp);
     int c = (p->tune.Bp == Bp && p->tune.scatter_bc != 0) ? p->tune.scatter_bc : dflt;
     if (!pull_choice_ok(p, c, Bp)) c = dflt;
     switch (c) {
@@ -4016,15 +4038,15 @@ static void gather_wt(Plan *p, float *img, int B, int Bp, float scale, hipStream
     }
 }
 
-template <int G, int NCH>
+template <int G, int NCH, int LB>
 static void gather_ta_n(Plan *p, float *img, int B, int Bp, float scale, hipStream_t s)
 {
-    const int nbc = (Bp + 63) / 64;
+    const int nbc = (Bp + LB - 1) / LB;
     const size_t lds = 0;   // static LDS
     const int bytes = (int)(sizeof(float) * ((size_t)p->D * p->geom.NB + 2) * Bp);
     const int tbytes = (int)(sizeof(int2) * (size_t)(p->Pd / 256) * p->D * 256);
     const int nwg = p->d_tord ? p->tile_launch : p->Pd / 256;
-    hipLaunchKernelGGL((k_gather_ta<G, NCH>), dim3(nwg, G * nbc), dim3(1024), lds, s, p->d_ttab, p->d_twin, p->d_pix,
+    hipLaunchKernelGGL((k_gather_ta<G, NCH, LB>), dim3(nwg, G * nbc), dim3(1024), lds, s, p->d_ttab, p->d_twin, p->d_pix,
                        p->d_bins, G > 1 ? p->d_gpart : img, p->D, p->geom.NB, p->P, B, Bp, scale, bytes, tbytes,
                        (const int32_t *)p->d_tord);
     if (G > 1) {
@@ -4034,13 +4056,13 @@ static void gather_ta_n(Plan *p, float *img, int B, int Bp, float scale, hipStre
     }
 }
 
-template <int G>
+template <int G, int LB = 64>
 static void gather_ta(Plan *p, float *img, int B, int Bp, float scale, hipStream_t s)
 {
     switch (p->tile_zr / 64) {   // 64-row rounds of the staged window (validity keeps it in 1..3)
-    case 1: gather_ta_n<G, 1>(p, img, B, Bp, scale, s); break;
-    case 2: gather_ta_n<G, 2>(p, img, B, Bp, scale, s); break;
-    default: gather_ta_n<G, 3>(p, img, B, Bp, scale, s); break;
+    case 1: gather_ta_n<G, 1, LB>(p, img, B, Bp, scale, s); break;
+    case 2: gather_ta_n<G, 2, LB>(p, img, B, Bp, scale, s); break;
+    default: gather_ta_n<G, 3, LB>(p, img, B, Bp, scale, s); break;
     }
 }
 
@@ -4152,7 +4174,8 @@ static const GatherVariant kGatherVariants[] = {{1, 8, 0},   {1, 4, 0},   {4, 4,
                                                 {0, -11, 4}, {0, -12, 1}, {0, -12, 2}, {0, -12, 4},
                                                 {0, -12, 8}, {0, -13, 1}, {0, -13, 2}, {0, -13, 4},
                                                 {0, -13, 8}, {0, -13, 16}, {0, -14, 4}, {0, -14, 8},
-                                                {0, -14, 16}, {0, -15, 4}, {0, -15, 8}, {0, -15, 16}};
+                                                {0, -14, 16}, {0, -15, 4}, {0, -15, 8}, {0, -15, 16},
+                                                {32, -16, 2}, {32, -16, 4}, {16, -16, 2}, {16, -16, 4}};
 constexpr int kNumGatherVariants = sizeof(kGatherVariants) / sizeof(kGatherVariants[0]);
 
 static bool gather_variant_ok(const Plan *p, int v, int Bp)
@@ -4173,8 +4196,8 @@ static bool gather_variant_ok(const Plan *p, int v, int Bp)
         if (p->D > kTaMaxD) return false;
         return g.lb == 1 || p->d_gpart;
     }
-    if (g.u == -10) {   // tile gather with asynchronous staging: three buffers of at most 3 rounds of 64 rows
-        if (p->use_sir || !p->d_ttab || Bp < 16 || p->tile_zr > 192) return false;
+    if (g.u == -10 || g.u == -16) {   // tile gather with asynchronous staging: three buffers of at most 3 rounds of 64 rows
+        if (p->use_sir || !p->d_ttab || Bp < (g.u == -10 ? 16 : 4) || p->tile_zr > 192) return false;
         if (sizeof(float) * ((size_t)p->D * p->geom.NB + 2) * Bp >= ((size_t)1 << 31)) return false;
         if (sizeof(int2) * (size_t)(p->Pd / 256) * p->D * 256 >= ((size_t)1 << 31)) return false;
         if (p->D > kTaMaxD) return false;
@@ -4223,6 +4246,18 @@ static int default_gather_variant(const Plan *p, int Bp)
     if (p->use_sir && Bp >= 16)
         for (int v : {39, 38, 37})   // SIR tile gather in four detector groups, two, one
             if (gather_variant_ok(p, v, Bp)) return v;
+    if (!p->use_sir && Bp >= 12 && Bp <= 64) {
+        // LDS tile gather with 32 sinograms per workgroup (16 up to Bp = 16) and two or more workgroups
+        // per CU, in two detector groups, four where those leave CUs without one.  Measured, stage time
+        // against the former choices: 301 x 333 x 28 0.29 / 1.22 ms (the 64-sinogram form 0.56), x 16
+        // 0.18 / 0.57 ms, x 12 0.18 / 0.43 ms (x 8: 0.17 / 0.13, so Bp = 8 stays), 400^2 x 64
+        // 0.74 / 0.84 ms (x 100: 2.4 / 1.7, so larger batches stay).
+        const bool small = Bp <= 16;
+        const int tiles = p->Pd / 256, chunks = small ? 1 : (Bp + 31) / 32;
+        const bool few = tiles * chunks * 2 < (small ? 1024 : 512);
+        const int v = small ? (few ? 58 : 57) : (few ? 56 : 55);
+        if (gather_variant_ok(p, v, Bp)) return v;
+    }
     if (Bp >= 64) {
         // LDS tile gathers in two detector groups (asynchronous, then register staging),
         // else the wave-uniform XCD gather
@@ -4295,7 +4330,11 @@ static int launch_gather(Plan *p, float *img, int B, int Bp, float scale, hipStr
     case 51: gather_ta1<16, 4, 2>(p, img, scale, s); break;
     case 52: gather_tp1<4>(p, img, scale, s); break;
     case 53: gather_tp1<8>(p, img, scale, s); break;
-    default: gather_tp1<16>(p, img, scale, s); break;
+    case 54: gather_tp1<16>(p, img, scale, s); break;
+    case 55: gather_ta<2, 32>(p, img, B, Bp, scale, s); break;
+    case 56: gather_ta<4, 32>(p, img, B, Bp, scale, s); break;
+    case 57: gather_ta<2, 16>(p, img, B, Bp, scale, s); break;
+    default: gather_ta<4, 16>(p, img, B, Bp, scale, s); break;
     }
     MBREC_HIP(hipGetLastError());
     return MBREC_OK;

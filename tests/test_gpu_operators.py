@@ -269,6 +269,32 @@ def test_autotuned_launch_matches_oracle(sir, B):
     assert rel_l2(xt.reshape(B, -1), xto) < TOL_OP, (gv, sc)
 
 
+@pytest.mark.parametrize("B", [9, 12, 13, 16, 17, 28, 32, 33, 48, 64, 65, 70])
+@pytest.mark.parametrize("smooth", [True, False])
+def test_default_batch_forms_match_oracle(B, smooth):
+    """The automatic forward and gather of a plan without SIR around the batch sizes where they
+    change (12, 16, 32, 64; several workgroups' columns), on an arc geometry whose tile windows
+    fit the LDS gather (its grid ends inside a tile in both directions) and on random travel
+    times, where the forms without windows run."""
+    import torch
+    _log(f"default batch forms B={B} smooth={smooth}")
+    if smooth:
+        m = _geometry_model(57, 70, 24, 700, 1e-4, sir=False, sigma=1.0)
+        plan, tt, R, shape = m.plan, _oracle_of(m).tt.T, _oracle_of(m).R, (70, 57)
+        D, nT = m.shape_sinogram
+    else:
+        D, nT, R, shape = 12, 160, 2.6666666666666665, (20, 23)
+        plan, tt, _, _ = _plan_problem(23, 20, D, nT, R, seed=70 + B)
+    x = rng(33).uniform(0, 1, (B, *shape))
+    sg = rng(34).standard_normal((B, D, nT))
+    yo = np.transpose(O.forward_das(x.reshape(B, -1), tt, nT, R), (0, 2, 1))
+    xto = O.transpose_das(np.transpose(sg, (0, 2, 1)), tt, R)
+    y = plan.forward(torch.tensor(x, dtype=torch.float32).cuda(), model=False).cpu().numpy()
+    xt = plan.transpose(torch.tensor(sg, dtype=torch.float32).cuda(), model=False).cpu().numpy()
+    assert rel_l2(y, yo) < TOL_OP
+    assert rel_l2(xt.reshape(B, -1), xto) < TOL_OP
+
+
 def test_one_sinogram_tile_variants_match_oracle():
     """Every one-sinogram tile form on a real arc geometry (the tile windows fit the LDS only
     for smooth travel times): forward choices 2, 3 (record streaming), 5, 6, 7 (tile form, thread
