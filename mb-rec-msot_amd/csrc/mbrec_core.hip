@@ -4,7 +4,10 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
+#include <atomic>
 #include <cstring>
+#include <system_error>
+#include <thread>
 #include <vector>
 #include <algorithm>
 
@@ -62,6 +65,21 @@ static void free_work(Plan *p)
     p->work_bytes = 0;
 }
 
+
+void keep_pool_scratch()
+{
+    static std::atomic<unsigned long long> warmed{0};
+    int dev = 0;
+    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 &&
+        !(warmed.fetch_or(1ull << dev) & (1ull << dev))) {
+        hipMemPool_t pool;
+        if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess) {
+            uint64_t keep = (uint64_t)1 << 30;
+            (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
+        }
+        (void)hipGetLastError();
+    }
+}
 
 int ensure_work(Plan *p, int B)
 {
@@ -404,6 +422,24 @@ static int build_sir_pull(Plan *p, const std::vector<int32_t> &slot_pix, const s
     return MBREC_OK;
 }
 
+// f(t) for t in [0, n) over a few threads
+template <class F>
+static void parallel_for(int n, F &&f)
+{
+    const int nt = std::max(1, std::min({n, 16, (int)std::thread::hardware_concurrency()}));
+    std::atomic<int> next{0};
+    auto work = [&]() {
+        for (int t; (t = next.fetch_add(1)) < n;) f(t);
+    };
+    std::vector<std::thread> th;
+    try {
+        for (int k = 1; k < nt; ++k) th.emplace_back(work);
+    } catch (const std::system_error &) {   // fewer threads than asked for: the ones there do it all
+    }
+    work();
+    for (auto &t : th) t.join();
+}
+
 // SIR transpose tables for the LDS tile form (d_stwin, d_stab): for pair (slot, d) with
 // decoded (nn, m, u) and window [s0, s0 + len) of its SIR index, the taps s whose sample
 // nn + s - Ls/2 lies in [0, nT + 2K) form [s_lo, s_hi); they read bin rows
@@ -429,8 +465,9 @@ static int build_sir_tiles(Plan *p, const std::vector<int32_t> &slot_pix, const 
     std::vector<int32_t> w((size_t)ntile * p->D, 0);
     std::vector<int4> tab((size_t)ntile * p->D * 256, make_int4(0, 0, 0, 0));
     const float scale = std::ldexp(1.0f, -g.F);
-    int wmax = 0;
-    for (int t = 0; t < ntile; ++t)
+    std::atomic<int> wmax_all{0};
+    parallel_for(ntile, [&](int t) {
+        int wmax = 0;
         for (int d = 0; d < p->D; ++d) {
             int lo = INT32_MAX, hi = INT32_MIN;
             int4 *e = tab.data() + ((size_t)t * p->D + d) * 256;
@@ -460,6 +497,10 @@ static int build_sir_tiles(Plan *p, const std::vector<int32_t> &slot_pix, const 
             for (int k = 0; k < 256; ++k)
                 if (e[k].w > 0) e[k].x -= lo;
         }
+        int seen = wmax_all;
+        while (wmax > seen && !wmax_all.compare_exchange_weak(seen, wmax)) {}
+    });
+    const int wmax = wmax_all;
     const int zr = 64 * ((wmax + 63) / 64);
     p->stile_wmax = wmax;
     if (zr > 256 || (size_t)p->Nsir_build * stride >= ((size_t)1 << 31)) return MBREC_OK;
@@ -469,6 +510,106 @@ static int build_sir_tiles(Plan *p, const std::vector<int32_t> &slot_pix, const 
         return rc;
     p->table_bytes += p->stab_bytes;
     p->stile_zr = zr;
+    return MBREC_OK;
+}
+
+// Tables of the matrix-core SIR transpose.  The pairs of a (tile, detector), sorted by phase and
+// first tap sample nf, are cut into groups of at most 16 of one phase whose taps in [0, nT + 2K)
+// lie in a window of 32 samples.  The window starts at the group's first such tap, moved back
+// where it would leave the staged samples [n_lo, n_lo + ns), and stays inside [0, nT + 2K), so that
+// the range check is the window's (a pair's offset points at its weight on the window's first
+// sample: the zero margins of d_sirw give the rest).  No tables where a (tile, detector) needs more
+// than 24 groups or 256 rows, or the axis is shorter than a window.
+static int build_sir_groups(Plan *p, const std::vector<int32_t> &slot_pix, const std::vector<int32_t> &tq,
+                            const int32_t *sidx, const int32_t *win, int Ls)
+{
+    const BinGeom &g = p->geom;
+    const int span = g.nT + 2 * g.K, half = Ls / 2, ntile = p->Pd / 256;
+    for (void *q : {(void *)p->d_sghdr, (void *)p->d_sgent, (void *)p->d_sgslot})
+        if (q) (void)hipFree(q);
+    p->table_bytes -= p->sg_bytes;
+    p->sg_bytes = 0;
+    p->d_sghdr = nullptr;
+    p->d_sgent = nullptr;
+    p->d_sgslot = nullptr;
+    p->sg_rows = 0;
+    int maxlen = 0;
+    for (int k = 0; k < p->Nsir_build; ++k) maxlen = std::max(maxlen, (int)win[2 * (size_t)k + 1]);
+    if (!p->d_sirw || maxlen > kSgWin || span < kSgWin) return MBREC_OK;
+    const int stride = maxlen + 2 * kSirWinPad;
+    const size_t ntd = (size_t)ntile * p->D;
+    std::vector<int32_t> hdr(ntd * 32, 0);
+    std::vector<int2> ent(ntd * kSgGroups * 16, make_int2(0, 0));
+    std::vector<uint32_t> slot(ntd * kSgGroups * 4, 0u);
+    const float scale = std::ldexp(1.0f, -g.F);
+    std::atomic<bool> fits{true};
+    std::atomic<int> ns_max{0};
+    parallel_for(ntile, [&](int t) {
+        struct Pair {
+            int key, nf, end, woff, slot;   // key: phase, then nf
+            float u;
+        };
+        Pair pr[256];
+        for (int d = 0; d < p->D && fits; ++d) {
+            int np = 0, lo = INT32_MAX, hi = 0;
+            for (int k = 0; k < 256; ++k) {
+                const size_t at = (size_t)d * p->Pd + (size_t)t * 256 + k;
+                if (slot_pix[(size_t)t * 256 + k] < 0 || tq[at] == INT32_MIN) continue;
+                const int sk = sidx[at], s0 = win[2 * (size_t)sk], len = win[2 * (size_t)sk + 1];
+                if (len <= 0) continue;
+                int nn, m;
+                host_decode(tq[at], g, nn, m);
+                const long long nf = (long long)nn + s0 - half;
+                if (nf + len <= 0 || nf >= span) continue;
+                const float fr = (float)(tq[at] & ((1 << g.F) - 1)) * scale;
+                const float u = m == 0 ? fr * g.iw0 : (m == 1 ? (fr - g.phi1) * g.iw1 : (fr - g.phi2) * g.iw2);
+                const int end = (int)std::min<long long>(nf + len, span);
+                pr[np++] = Pair{(m << 24) + (int)nf + 4096, (int)nf, end, (int)((size_t)sk * stride + kSirWinPad), k, u};
+                lo = std::min(lo, std::max((int)nf, 0));
+                hi = std::max(hi, end);
+            }
+            const size_t td = (size_t)t * p->D + d;
+            int32_t *h = &hdr[td * 32];
+            if (!np) continue;
+            std::sort(pr, pr + np, [](const Pair &a, const Pair &b) { return a.key != b.key ? a.key < b.key : a.slot < b.slot; });
+            if (hi - lo < kSgWin) {   // at least a window, inside the axis
+                lo = std::min(lo, span - kSgWin);
+                hi = std::max(hi, lo + kSgWin);
+            }
+            int seen = ns_max;
+            while (hi - lo > seen && !ns_max.compare_exchange_weak(seen, hi - lo)) {}
+            int ng = 0;
+            for (int i = 0; i < np;) {
+                const int m = pr[i].key >> 24, n0 = std::min(std::max(pr[i].nf, 0), hi - kSgWin);
+                int cnt = 0;
+                if (ng == kSgGroups) {
+                    fits = false;
+                    break;
+                }
+                while (i + cnt < np && cnt < 16 && (pr[i + cnt].key >> 24) == m && pr[i + cnt].end - n0 <= kSgWin) ++cnt;
+                for (int k = 0; k < cnt; ++k) {
+                    const Pair &q = pr[i + k];
+                    int32_t ub;
+                    std::memcpy(&ub, &q.u, sizeof(ub));
+                    ent[(td * kSgGroups + ng) * 16 + k] = make_int2(q.woff + n0 - q.nf, ub);
+                    slot[(td * kSgGroups + ng) * 4 + k / 4] |= (uint32_t)q.slot << 8 * (k % 4);
+                }
+                h[2 + ng++] = (n0 - lo) | (m << 8) | (cnt << 16);
+                i += cnt;
+            }
+            h[0] = lo;
+            h[1] = ng;
+        }
+    });
+    const int rows = 64 * ((3 * ns_max + 1 + 63) / 64);
+    if (!fits || rows > 256 || !ns_max) return MBREC_OK;
+    int rc;
+    if ((rc = dalloc(&p->d_sghdr, hdr.size(), &p->sg_bytes)) || (rc = dalloc(&p->d_sgent, ent.size(), &p->sg_bytes)) ||
+        (rc = dalloc(&p->d_sgslot, slot.size(), &p->sg_bytes)) || (rc = upload(p->d_sghdr, hdr.data(), hdr.size())) ||
+        (rc = upload(p->d_sgent, ent.data(), ent.size())) || (rc = upload(p->d_sgslot, slot.data(), slot.size())))
+        return rc;
+    p->table_bytes += p->sg_bytes;
+    p->sg_rows = rows;
     return MBREC_OK;
 }
 
@@ -762,7 +903,7 @@ static int build_tile_windows(Plan *p, const std::vector<int32_t> &tq)
 static void free_plan(Plan *p)
 {
     void *ptrs[] = {p->d_pix, p->d_tq, p->d_sidx, p->d_sir, p->d_swin, p->d_ir, p->d_irf, p->d_ir64, p->d_irf64,
-                    p->d_kz,  p->d_kx, p->d_rec, p->d_rec_off, p->d_rec_k, p->d_rec1, p->d_twin, p->d_ptab, p->d_ttab, p->d_srec, p->d_srec_off, p->d_sirw, p->d_stwin, p->d_stab,
+                    p->d_kz,  p->d_kx, p->d_rec, p->d_rec_off, p->d_rec_k, p->d_rec1, p->d_twin, p->d_ptab, p->d_ttab, p->d_srec, p->d_srec_off, p->d_sirw, p->d_stwin, p->d_stab, p->d_sghdr, p->d_sgent, p->d_sgslot,
                     p->d_tfrec, p->d_tfroff, p->d_tfdesc, p->d_tfpart, p->d_tfsrec, p->d_tfsro, p->d_tq1, p->d_tord};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
@@ -910,6 +1051,7 @@ int mbrec_plan_set_sir(mbrec_plan h, const int32_t *sirIdx, const double *sir, i
         p->Nsir_build = Nsir;
         if ((rc = build_sir_pull(p, slot_pix, tq, sidx.data(), win.data(), Ls, sirf.data()))) return rc;
         if ((rc = build_sir_tiles(p, slot_pix, tq, sidx.data(), win.data(), Ls))) return rc;
+        if ((rc = build_sir_groups(p, slot_pix, tq, sidx.data(), win.data(), Ls))) return rc;
     }
     p->use_sir = 1;
     p->Ls = Ls;

@@ -44,6 +44,9 @@ constexpr int kSirBandTS = 32;   // samples per wave of the band-form SIR forwar
 constexpr int kSirBandShift = 8, kSirBandRun = 4;
 static inline int sband_rows(int rb) { return rb > 1 ? kSirBandShift * rb + 24 : kSirBandTS; }
 
+// groups of a (tile, detector) in the matrix-core SIR transpose, samples of a group's window
+constexpr int kSgGroups = 24, kSgWin = 32;
+
 struct BinGeom {
     float phi1, phi2;            // sorted interior breakpoint phases in [0,1)
     float iw0, iw1, iw2;         // 1 / segment widths (0 for empty segments)
@@ -126,6 +129,16 @@ struct Plan {
     int stile_zr = 0;            // staged rows: 64 * ceil(longest window / 64)
     int stile_wmax = 0;          // longest window
     size_t stab_bytes = 0;
+    // SIR transpose on the matrix cores: per (256-slot tile, detector) the pairs in groups of at
+    // most 16 with one phase whose in-range taps lie in 32 samples (see build_sir_groups):
+    // d_sghdr [32] = {first staged sample, groups, per group (window start from it | phase << 8 |
+    // pairs << 16)}, d_sgent [24][16] = (d_sirw offset of the window start, u bits),
+    // d_sgslot [24][4] = the pairs' slots, four to a word
+    int32_t *d_sghdr = nullptr;
+    int2 *d_sgent = nullptr;
+    uint32_t *d_sgslot = nullptr;
+    int sg_rows = 0;             // staged bin rows: 64 * ceil(longest / 64)
+    size_t sg_bytes = 0;
     int32_t *d_srec_off = nullptr;
     int sp_lo = 0, sp_n = 0, Nsir_build = 0;
     size_t srec_bytes = 0;
@@ -165,6 +178,12 @@ struct Plan {
     int pins = 0;                // batches whose captured graphs use this plan's buffers
     TuneChoice tune;
 };
+
+// Keeps up to 1 GB of released stream-ordered scratch in the current device's default pool between
+// calls, so that a call's allocations do not map fresh memory each time (once per device; the
+// pool's own ordering makes the memory safe to share between streams and threads).  1 GB holds
+// the TV prox of 32 images of 600^2 (0.65 GB), whose hipMalloc / hipFree took 1.5 ms a call.
+void keep_pool_scratch();
 
 static inline int batch_stride(int B) { return B <= 1 ? 1 : (B + 3) / 4 * 4; }
 

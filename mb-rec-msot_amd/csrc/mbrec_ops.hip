@@ -2824,6 +2824,170 @@ __global__ __launch_bounds__(1024) void k_gather_tas(const int4 *__restrict__ st
     }
 }
 
+// SIR transpose for batches on the FP32 matrix cores: WG = 8 waves, one 256-slot tile x
+// LB = 16 NCB sinograms x one of G detector groups.  The tile's pairs with a detector come in
+// groups of at most 16 that share a phase and a window of 32 samples (build_sir_groups), so a
+// group is a product [16 pairs x 32 samples] x [32 samples x LB] of weights and bins, once with
+// weights w (1 - u) and the phase's bin rows and once with w u and the next rows, summed in
+// one accumulator: 16 NCB products 16x16x4.  The sample order is free: lane group q holds samples
+// 8 q + 0..7, so a pair's weights are two 16-byte loads per lane (4-byte aligned); odd lane
+// groups take them in swapped pairs, which puts their bin rows on the other 32 LDS banks.
+// Per detector the tile's bin rows are copied memory -> LDS once; the results go to the pixels'
+// sums in LDS (every pixel once per detector), which move to registers every eight detectors.
+// Two workgroups share a CU, one waiting for its rows and weights while the other multiplies.
+// Bound by the matrix cores: about 18 groups of 1024 cycles (NCB = 2) per tile and detector, at
+// 400^2 x 64 2.4 of 4.3 ms; the rest is the two barriers per detector.  Gather stage against the
+// vector form k_gather_tas (two FMAs and two lane reads per tap; it remains for windows that do
+// not fit the groups): 400^2 x 64 7.7 -> 4.3 ms, 300^2 x 28 4.3 -> 1.33 ms, x 4 1.66 (record lanes)
+// -> 0.80 ms.  The XCD order cut L2 misses from 26 to 8 GB at 400^2 x 64 (4.7 -> 4.5 ms).
+template <int G, int NCH, int NCB>
+__global__ __launch_bounds__(512, 4) void k_gather_sg(const int32_t *__restrict__ hdr, const int2 *__restrict__ ent,
+                                                      const uint32_t *__restrict__ slots,
+                                                      const int32_t *__restrict__ pix, const float *__restrict__ bins,
+                                                      const float *__restrict__ sirw, float *__restrict__ out,
+                                                      const int32_t *__restrict__ tord, int ntile, int tlen, int nbc,
+                                                      int D, int NB, int P, int B, int Bp, float scale)
+{
+    constexpr int LB = 16 * NCB, ROWS = 64 * NCH, RPL = 256 / LB, NV = 256 * LB / 512, GW = kSgGroups / 8;
+    __shared__ __attribute__((aligned(16))) float s_row[ROWS * LB];
+    __shared__ float s_acc[257 * LB];
+    // blocks of an XCD (every eighth): the column chunks of a tile side by side, then the next tile of
+    // the XCD's compact run, then the next detector group
+    const int r_ = blockIdx.x >> 3, tj = (r_ / nbc) % tlen, b0 = (r_ % nbc) * LB, grp = r_ / nbc / tlen;
+    const int ti = tj * 8 + (blockIdx.x & 7), tile = tord ? tord[ti] : ti < ntile ? ti : -1;
+    if (tile < 0) return;   // whole workgroup, before any barrier
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, q = lane >> 4, odd = q & 1;
+    const int DG = (D + G - 1) / G, dbeg = grp * DG, dend = min(D, dbeg + DG);
+    const int last_row = D * NB + 1;   // of the bins (two zero rows after the detectors')
+    const int lrow = lane / (LB / 4), lcol = min(b0 + 4 * (lane % (LB / 4)), Bp - 4);   // staging: row of a load, columns
+    float tot[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        tot[k] = 0.0f;
+        s_acc[tid + 512 * k] = 0.0f;
+    }
+    int2 e[GW];
+    uint32_t sl[GW];
+    auto entries = [&](int d) __attribute__((always_inline)) {
+        const size_t g0 = ((size_t)tile * D + d) * kSgGroups + wv;
+#pragma unroll
+        for (int k = 0; k < GW; ++k) {
+            e[k] = ent[(g0 + 8 * k) * 16 + i];
+            sl[k] = slots[(g0 + 8 * k) * 4 + q];
+        }
+    };
+    if (dbeg < dend) entries(dbeg);
+    for (int d = dbeg; d < dend; ++d) {
+        const int32_t *h = hdr + ((size_t)tile * D + d) * 32;
+        const int ng = h[1];
+        __syncthreads();   // the rows of the previous detector are no longer read
+        const int row0 = d * NB + 3 * h[0];
+#pragma unroll
+        for (int c = 0; c < (ROWS / RPL + 7) / 8; ++c) {
+            const int r0 = RPL * (8 * c + wv);
+            if (r0 < ROWS)
+                __builtin_amdgcn_global_load_lds(
+                    (const __attribute__((address_space(1))) void *)(bins + (size_t)min(row0 + r0 + lrow, last_row) * Bp +
+                                                                     lcol),
+                    (__attribute__((address_space(3))) void *)(s_row + r0 * LB), 16, 0, 0);
+        }
+        // weights of this wave's groups (absent groups read the table's start)
+        f32x4u w[GW][2];
+        float u[GW];
+        uint32_t slc[GW];
+#pragma unroll
+        for (int k = 0; k < GW; ++k) {
+            const f32x4u *wp = reinterpret_cast<const f32x4u *>(sirw + e[k].x + 8 * q);
+            w[k][0] = wp[0];
+            w[k][1] = wp[1];
+            u[k] = __int_as_float(e[k].y);
+            slc[k] = sl[k];
+        }
+        __builtin_amdgcn_s_waitcnt(kWaitVm(0));
+        __syncthreads();
+        if (d + 1 < dend) entries(d + 1);
+#pragma unroll
+        for (int k = 0; k < GW; ++k) {
+            const int g = wv + 8 * k;
+            if (g >= ng) break;   // uniform
+            const int gh = h[2 + g], cnt = gh >> 16;
+            const float u0 = 1.0f - u[k], u1 = u[k];
+            // LDS row of lane group q's sample 8 q (+ 1 for odd groups, whose sample order is swapped in pairs)
+            const float *row = s_row + (3 * ((gh & 255) + 8 * q) + ((gh >> 8) & 255)) * LB + i;
+            const float *re = row + odd * 3 * LB, *ro = row + (1 - odd) * 3 * LB;
+            f32x4 acc[NCB];
+#pragma unroll
+            for (int c = 0; c < NCB; ++c) acc[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            // bin rows of four samples at a time, the next four in flight during their products (the barriers
+            // keep the compiler from moving every read next to its product)
+            float rv[2][4][2][NCB];
+            auto read = [&](int hf) __attribute__((always_inline)) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int s = 4 * hf + t;
+                    const float *r = ((s & 1) ? ro : re) + 3 * (s & 6) * LB;
+#pragma unroll
+                    for (int c = 0; c < NCB; ++c) {
+                        rv[hf][t][0][c] = r[16 * c];
+                        rv[hf][t][1][c] = r[LB + 16 * c];
+                    }
+                }
+            };
+            auto mul = [&](int hf) __attribute__((always_inline)) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const float wa = w[k][hf][t], wb = w[k][hf][t ^ 1], ws = odd ? wb : wa;
+                    const float a0 = ws * u0, a1 = ws * u1;
+#pragma unroll
+                    for (int c = 0; c < NCB; ++c)
+                        acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, rv[hf][t][0][c], acc[c], 0, 0, 0);
+#pragma unroll
+                    for (int c = 0; c < NCB; ++c)
+                        acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, rv[hf][t][1][c], acc[c], 0, 0, 0);
+                }
+            };
+            read(0);
+            read(1);
+            __builtin_amdgcn_sched_barrier(0);
+            mul(0);
+            mul(1);
+            __builtin_amdgcn_sched_barrier(0);
+            // lane: sinogram i (+ 16 c), pairs 4 q + r (past the group's end: to a row that nobody reads)
+            float *px[4], pv[4][NCB];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                px[r] = s_acc + (4 * q + r < cnt ? (slc[k] >> 8 * r) & 255 : 256) * LB + i;
+#pragma unroll
+                for (int c = 0; c < NCB; ++c) pv[r][c] = px[r][16 * c];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int c = 0; c < NCB; ++c) px[r][16 * c] = pv[r][c] + acc[c][r];
+        }
+        if (((d - dbeg) & 7) == 7 || d + 1 == dend) {
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {   // read and cleared by the same thread, before the barriers of the next detector
+                tot[k] += s_acc[tid + 512 * k];
+                s_acc[tid + 512 * k] = 0.0f;
+            }
+        }
+    }
+    const int b = b0 + tid % LB;
+    if (b >= B) return;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const int px = pix[(size_t)tile * 256 + tid / LB + (512 / LB) * k];
+        if (px < 0) continue;
+        if (G > 1)
+            out[((size_t)grp * B + b) * P + px] = tot[k];
+        else
+            out[(size_t)b * P + px] = scale * tot[k];
+    }
+}
+
 // Transpose without SIR for one sinogram, LDS tile form: WG = one 256-slot tile (thread k:
 // slot k) x one of G detector groups.  The group's window origins go to LDS first; per
 // detector the tile's bin window (at most tile_zr <= 256 rows; one row per thread) is
@@ -4093,6 +4257,30 @@ static void gather_tas(Plan *p, float *img, int B, int Bp, float scale, hipStrea
     }
 }
 
+template <int G, int NCH, int NCB>
+static void gather_sg_n(Plan *p, float *img, int B, int Bp, float scale, hipStream_t s)
+{
+    const int nbc = (Bp + 16 * NCB - 1) / (16 * NCB), ntile = p->Pd / 256;
+    const int tlen = p->d_tord ? p->tile_launch / 8 : (ntile + 7) / 8;   // tiles per XCD
+    hipLaunchKernelGGL((k_gather_sg<G, NCH, NCB>), dim3(8 * tlen * G * nbc), dim3(512), 0, s, p->d_sghdr, p->d_sgent,
+                       p->d_sgslot, p->d_pix, p->d_bins, p->d_sirw, p->d_gpart, (const int32_t *)p->d_tord, ntile, tlen, nbc,
+                       p->D, p->geom.NB, p->P, B, Bp, scale);
+    const size_t n = (size_t)B * p->P;
+    hipLaunchKernelGGL(k_sum_parts<G>, dim3(std::min<size_t>(4096, (n + 255) / 256)), dim3(256), 0, s,
+                       (const float *)p->d_gpart, img, n, scale);
+}
+
+template <int G, int NCB>
+static void gather_sg(Plan *p, float *img, int B, int Bp, float scale, hipStream_t s)
+{
+    switch (p->sg_rows / 64) {
+    case 1:
+    case 2: gather_sg_n<G, 2, NCB>(p, img, B, Bp, scale, s); break;
+    case 3: gather_sg_n<G, 3, NCB>(p, img, B, Bp, scale, s); break;
+    default: gather_sg_n<G, 4, NCB>(p, img, B, Bp, scale, s); break;
+    }
+}
+
 template <int G>
 static void gather_tp1(Plan *p, float *img, float scale, hipStream_t s)
 {
@@ -4175,7 +4363,8 @@ static const GatherVariant kGatherVariants[] = {{1, 8, 0},   {1, 4, 0},   {4, 4,
                                                 {0, -12, 8}, {0, -13, 1}, {0, -13, 2}, {0, -13, 4},
                                                 {0, -13, 8}, {0, -13, 16}, {0, -14, 4}, {0, -14, 8},
                                                 {0, -14, 16}, {0, -15, 4}, {0, -15, 8}, {0, -15, 16},
-                                                {32, -16, 2}, {32, -16, 4}, {16, -16, 2}, {16, -16, 4}};
+                                                {32, -16, 2}, {32, -16, 4}, {16, -16, 2}, {16, -16, 4},
+                                                {32, -17, 4}, {32, -17, 8}, {16, -17, 4}, {16, -17, 8}};
 constexpr int kNumGatherVariants = sizeof(kGatherVariants) / sizeof(kGatherVariants[0]);
 
 static bool gather_variant_ok(const Plan *p, int v, int Bp)
@@ -4190,6 +4379,8 @@ static bool gather_variant_ok(const Plan *p, int v, int Bp)
     if (g.u == -12)   // SIR tile gather for one sinogram: the SIR tile tables, G partial images
         return p->use_sir && p->d_stab && p->stile_zr >= 64 && p->stile_zr <= 256 && Bp == 1 &&
                (g.lb == 1 || p->d_gpart);
+    if (g.u == -17)   // matrix-core SIR gather: tables built
+        return p->use_sir && p->d_sghdr && p->sg_rows >= 64 && p->sg_rows <= 256 && Bp >= 4 && p->d_gpart;
     if (g.u == -11) {   // SIR tile gather: tables built, window within 4 rounds of 64 rows, 32-bit offsets
         if (!p->use_sir || !p->d_stab || p->stile_zr < 64 || p->stile_zr > 256 || Bp < 16) return false;
         if (sizeof(float) * ((size_t)p->D * p->geom.NB + 2) * Bp >= ((size_t)1 << 31)) return false;
@@ -4243,6 +4434,7 @@ static int default_gather_variant(const Plan *p, int Bp)
                    // in 16, then the decoding form in 8), else record-lane
         for (int v : {43, 54, 47, 0})
             if (gather_variant_ok(p, v, Bp)) return v;
+    if (p->use_sir && Bp >= 4 && gather_variant_ok(p, 59, Bp)) return Bp <= 16 ? 61 : 59;
     if (p->use_sir && Bp >= 16)
         for (int v : {39, 38, 37})   // SIR tile gather in four detector groups, two, one
             if (gather_variant_ok(p, v, Bp)) return v;
@@ -4334,7 +4526,11 @@ static int launch_gather(Plan *p, float *img, int B, int Bp, float scale, hipStr
     case 55: gather_ta<2, 32>(p, img, B, Bp, scale, s); break;
     case 56: gather_ta<4, 32>(p, img, B, Bp, scale, s); break;
     case 57: gather_ta<2, 16>(p, img, B, Bp, scale, s); break;
-    default: gather_ta<4, 16>(p, img, B, Bp, scale, s); break;
+    case 58: gather_ta<4, 16>(p, img, B, Bp, scale, s); break;
+    case 59: gather_sg<4, 2>(p, img, B, Bp, scale, s); break;
+    case 60: gather_sg<8, 2>(p, img, B, Bp, scale, s); break;
+    case 61: gather_sg<4, 1>(p, img, B, Bp, scale, s); break;
+    default: gather_sg<8, 1>(p, img, B, Bp, scale, s); break;
     }
     MBREC_HIP(hipGetLastError());
     return MBREC_OK;

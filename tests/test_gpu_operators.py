@@ -243,6 +243,48 @@ def test_sir_forward_band_edges(length, B):
     assert np.abs(y - yo).max() < 1e-4 * np.abs(yo).max()
 
 
+@pytest.mark.parametrize("B", [2, 4, 13, 16, 17, 28, 33, 70])
+@pytest.mark.parametrize("crop", ["inside", "start", "end"])
+def test_sir_transpose_groups_match_oracle(B, crop):
+    """The matrix-core SIR transpose on an arc geometry (grid ending inside tiles, batches around
+    16 and 32 columns), with every tap on the sample axis and with travel times that leave it at
+    its start or end, where the groups' windows are moved back and taps drop out; empty
+    windows among the SIR entries."""
+    import torch
+    from mbrec.model import DevicePlan
+    Nz, Nx, D, R, Ls = 37, 53, 9, 2.6666666666666665, 31
+    _log(f"sir groups B={B} crop={crop}")
+    tt = geometry_tt(Nz, Nx, 1e-4, D, 0.01, 160.0, 1500.0, 4e7).reshape(D, -1)
+    lo, hi = int(tt.min()), int(tt.max()) + 1
+    nT = hi - lo + 60
+    tt = tt - lo + {"inside": 30, "start": -50, "end": 130}[crop]
+    g = rng(900)
+    nsir = 40
+    sir = g.standard_normal((Ls, nsir))
+    se = np.zeros((2, nsir), dtype=np.int32)
+    for k in range(nsir):
+        n = int(g.integers(14, 25))
+        s0 = int(g.integers(3, 6))
+        se[:, k] = (s0, s0 + n - 1)
+    se[:, 0] = (3, 2)
+    sidx = g.integers(1, nsir + 1, size=(Nz * Nx, D)).astype(np.int32)
+    plan = DevicePlan(Nz, Nx, D, nT, R, tt, sir=(np.ascontiguousarray(sidx.T), np.ascontiguousarray(sir.T),
+                                                 np.ascontiguousarray(se.T)))
+    sg = g.standard_normal((B, D, nT))
+    xto = O.transpose_sir(np.transpose(sg, (0, 2, 1)), sidx, np.ascontiguousarray(tt.T), sir, se, R)
+    sd = torch.tensor(sg, dtype=torch.float32).cuda()
+    ran = 0
+    for v in (-1, 59, 60, 61, 62):
+        try:
+            plan.set_launch(B, v, 0)
+        except Exception:
+            continue
+        ran += v > 0
+        xt = plan.transpose(sd, model=False).cpu().numpy()
+        assert rel_l2(xt.reshape(B, -1), xto) < TOL_OP, v
+    assert ran == 4      # the geometry's pairs fit the groups
+
+
 @pytest.mark.parametrize("sir", [False, True])
 @pytest.mark.parametrize("B", [1, 64])
 def test_autotuned_launch_matches_oracle(sir, B):
