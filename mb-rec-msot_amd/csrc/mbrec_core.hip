@@ -5,6 +5,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <atomic>
+#include <mutex>
 #include <cstring>
 #include <system_error>
 #include <thread>
@@ -65,20 +66,41 @@ static void free_work(Plan *p)
     p->work_bytes = 0;
 }
 
+static std::mutex g_pool_mu;
+static hipMemPool_t g_pool[kPoolDevices];
 
-void keep_pool_scratch()
+hipError_t scratch_malloc(void **p, size_t bytes, hipStream_t s)
 {
-    static std::atomic<unsigned long long> warmed{0};
     int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 &&
-        !(warmed.fetch_or(1ull << dev) & (1ull << dev))) {
-        hipMemPool_t pool;
-        if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess) {
-            uint64_t keep = (uint64_t)1 << 30;
-            (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    hipMemPool_t pool = nullptr;
+    if (dev >= 0 && dev < kPoolDevices) {
+        std::lock_guard<std::mutex> lk(g_pool_mu);
+        if (!g_pool[dev]) {
+            hipMemPoolProps pr{};
+            pr.allocType = hipMemAllocationTypePinned;
+            pr.location.type = hipMemLocationTypeDevice;
+            pr.location.id = dev;
+            if (hipMemPoolCreate(&g_pool[dev], &pr) == hipSuccess) {
+                uint64_t keep = kPoolKeep;
+                (void)hipMemPoolSetAttribute(g_pool[dev], hipMemPoolAttrReleaseThreshold, &keep);
+            } else {
+                g_pool[dev] = nullptr;
+                (void)hipGetLastError();
+            }
         }
-        (void)hipGetLastError();
+        pool = g_pool[dev];
     }
+    return pool ? hipMallocFromPoolAsync(p, bytes, pool, s) : hipMallocAsync(p, bytes, s);
+}
+
+void scratch_trim()
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kPoolDevices) return;
+    std::lock_guard<std::mutex> lk(g_pool_mu);
+    if (g_pool[dev] && hipMemPoolTrimTo(g_pool[dev], 0) != hipSuccess) (void)hipGetLastError();
 }
 
 int ensure_work(Plan *p, int B)
@@ -1136,6 +1158,7 @@ int mbrec_plan_destroy(mbrec_plan h)
     if (h->p.pins) return set_error(MBREC_ERR_ARG, "mbrec:planPinned", "plan is held by a batch graph");
     (void)hipDeviceSynchronize();
     free_plan(&h->p);
+    scratch_trim();
     delete h;
     return MBREC_OK;
 }

@@ -31,16 +31,13 @@
 namespace mbrec {
 
 // ---- TV prox kernels (images [B][Nx][Nz] column-major = z fastest) -------------
-// g = (double) z
-__global__ void k_tv_load(const float *__restrict__ z, double *__restrict__ g, double *__restrict__ u,
-                          double *__restrict__ bz, double *__restrict__ bx, double *__restrict__ dz,
-                          double *__restrict__ dx, size_t n)
+// u = (double) z, b = q = 0
+__global__ void k_tv_load(const float *__restrict__ z, double *__restrict__ u, double *__restrict__ bz,
+                          double *__restrict__ bx, double *__restrict__ qz, double *__restrict__ qx, size_t n)
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const double v = z[i];
-        g[i] = v;
-        u[i] = v;
-        bz[i] = bx[i] = dz[i] = dx[i] = 0.0;
+        u[i] = z[i];
+        bz[i] = bx[i] = qz[i] = qx[i] = 0.0;
     }
 }
 
@@ -48,6 +45,7 @@ __global__ void k_tv_load(const float *__restrict__ z, double *__restrict__ g, d
 constexpr int kNmMaxFactors = 24;
 constexpr int kNmLdsPoints = 2048;   // complex points per LDS buffer (two buffers: 64 KB)
 constexpr int kNmMaxN = kNmLdsPoints;
+constexpr int kNmIpPoints = 4096;    // complex points of an in-place transform (one buffer)
 
 struct NmFactors {
     int n;
@@ -117,6 +115,140 @@ __device__ double2 *nm_fft(double2 *a, double2 *b, int N, int C, const NmFactors
     return a;
 }
 
+// The same transform in place for N a product of 2, 3, 4, 5, 7 and 8: a thread takes whole
+// butterflies (p points read once, twiddled, transformed in registers), all reads of a stage before
+// its writes.  Against a thread per output (p reads and p twiddles each, two LDS buffers) the
+// passes of a 600^2 x 32 solve take 0.27 instead of 0.51 ms.  At most 4096 points for 512 threads (2048 for
+// 256), so KB butterflies per thread cover a stage.
+__device__ __forceinline__ double2 nm_mul(double2 x, double2 w) { return make_double2(x.x * w.x - x.y * w.y, x.x * w.y + x.y * w.x); }
+__device__ __forceinline__ double2 nm_add(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ double2 nm_sub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
+// -i sg x
+__device__ __forceinline__ double2 nm_rot(double2 x, double sg) { return make_double2(sg * x.y, -sg * x.x); }
+
+// x_q <- sum_r x_r e^{-2 pi i sg q r / P}
+template <int P>
+__device__ __forceinline__ void nm_dft(double2 (&x)[P], double sg)
+{
+    if constexpr (P == 2) {
+        const double2 t = x[0];
+        x[0] = nm_add(t, x[1]);
+        x[1] = nm_sub(t, x[1]);
+    } else if constexpr (P == 4) {
+        const double2 a = nm_add(x[0], x[2]), b = nm_sub(x[0], x[2]), c = nm_add(x[1], x[3]);
+        const double2 d = nm_rot(nm_sub(x[1], x[3]), sg);
+        x[0] = nm_add(a, c);
+        x[1] = nm_add(b, d);
+        x[2] = nm_sub(a, c);
+        x[3] = nm_sub(b, d);
+    } else if constexpr (P == 8) {
+        double2 e[4] = {x[0], x[2], x[4], x[6]}, o[4] = {x[1], x[3], x[5], x[7]};
+        nm_dft<4>(e, sg);
+        nm_dft<4>(o, sg);
+        constexpr double h = 0.70710678118654752440;
+        o[1] = nm_mul(o[1], make_double2(h, -sg * h));
+        o[2] = nm_rot(o[2], sg);
+        o[3] = nm_mul(o[3], make_double2(-h, -sg * h));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            x[k] = nm_add(e[k], o[k]);
+            x[k + 4] = nm_sub(e[k], o[k]);
+        }
+    } else {   // odd: sums and differences of x_r and x_{P - r}
+        constexpr int H = (P - 1) / 2;
+        constexpr double c[4] = {1.0, P == 3 ? -0.5 : P == 5 ? 0.30901699437494742410 : 0.62348980185873353053,
+                                 P == 5 ? -0.80901699437494742410 : -0.22252093395631440429, -0.90096886790241912624};
+        constexpr double n[4] = {0.0, P == 3 ? 0.86602540378443864676 : P == 5 ? 0.95105651629515357212 : 0.78183148246802980871,
+                                 P == 5 ? 0.58778525229247312917 : 0.97492791218182360702, 0.43388373911755812048};
+        double2 sm[H], df[H], y0 = x[0];
+#pragma unroll
+        for (int r = 1; r <= H; ++r) {
+            sm[r - 1] = nm_add(x[r], x[P - r]);
+            df[r - 1] = nm_sub(x[r], x[P - r]);
+            y0 = nm_add(y0, sm[r - 1]);
+        }
+        const double2 x0 = x[0];
+        x[0] = y0;
+#pragma unroll
+        for (int q = 1; q <= H; ++q) {
+            double2 A = x0, B = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int r = 1; r <= H; ++r) {
+                const int t = q * r % P, k = t <= H ? t : P - t;
+                const double cs = c[k], sn = t <= H ? n[k] : -n[k];
+                A.x += cs * sm[r - 1].x;
+                A.y += cs * sm[r - 1].y;
+                B.x += sn * df[r - 1].x;
+                B.y += sn * df[r - 1].y;
+            }
+            const double2 R = nm_rot(B, sg);
+            x[q] = nm_add(A, R);
+            x[P - q] = nm_sub(A, R);
+        }
+    }
+}
+
+template <int P, int KB>
+__device__ __forceinline__ void nm_stage(double2 *a, int N, int C, int Ns, const double2 *__restrict__ tw, bool inverse)
+{
+    const int m = N / P, step = m / Ns, total = C * m;
+    const float invm = 1.0f / (float)m, invNs = 1.0f / (float)Ns;
+    const double sg = inverse ? -1.0 : 1.0;
+    double2 x[KB][P];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+        const int o = threadIdx.x + kb * blockDim.x;
+        if (o < total) {
+            int c, j, jn, k;
+            divmod_small(o, m, invm, c, j);
+            divmod_small(j, Ns, invNs, jn, k);
+            const double2 *src = a + c * N + j;
+#pragma unroll
+            for (int r = 0; r < P; ++r) x[kb][r] = src[r * m];
+            if (Ns > 1) {
+#pragma unroll
+                for (int r = 1; r < P; ++r) {
+                    const double2 w = tw[r * k * step];
+                    x[kb][r] = nm_mul(x[kb][r], make_double2(w.x, sg * w.y));
+                }
+            }
+            nm_dft<P>(x[kb], sg);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+        const int o = threadIdx.x + kb * blockDim.x;
+        if (o < total) {
+            int c, j, jn, k;
+            divmod_small(o, m, invm, c, j);
+            divmod_small(j, Ns, invNs, jn, k);
+            double2 *dst = a + c * N + jn * Ns * P + k;
+#pragma unroll
+            for (int q = 0; q < P; ++q) dst[q * Ns] = x[kb][q];
+        }
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ void nm_fft_ip(double2 *a, int N, int C, const NmFactors &f, const double2 *__restrict__ tw,
+                                          bool inverse)
+{
+    int Ns = 1;
+    for (int s = 0; s < f.n; ++s) {
+        const int p = f.p[s];
+        switch (p) {   // uniform
+        case 2: nm_stage<2, 4>(a, N, C, Ns, tw, inverse); break;
+        case 3: nm_stage<3, 3>(a, N, C, Ns, tw, inverse); break;
+        case 4: nm_stage<4, 2>(a, N, C, Ns, tw, inverse); break;
+        case 5: nm_stage<5, 2>(a, N, C, Ns, tw, inverse); break;
+        case 7: nm_stage<7, 2>(a, N, C, Ns, tw, inverse); break;
+        default: nm_stage<8, 1>(a, N, C, Ns, tw, inverse); break;
+        }
+        Ns *= p;
+    }
+}
+
 // Orthonormal DCT-II of the two real rows packed in Z = FFT(v1 + i v2) (v the reordered
 // rows): X_a[k] = s_k Re(e^{-i pi k/2N} V_a[k]), V1 = (Z[k] + conj Z[N-k]) / 2,
 // V2 = (Z[k] - conj Z[N-k]) / 2i; s_0 = sqrt(1/N), s_k = sqrt(2/N).
@@ -152,13 +284,15 @@ struct NmArgs {
     const double *lam;
 };
 
-// Pass 1, along z: rows = pairs of image columns (ix, ix + 1), loaded as the right-hand
-// side rhs = g - B'(b - d),
+// Pass 1, along z: rows = pairs of image columns (ix, ix + 1), loaded as the right-hand side
+// rhs = g - B' q with q = b - d,
 //   (B' v)(iz,ix) = vz(iz,ix)[iz>0] - vz(iz+1,ix)[iz+1<N] + vx(iz,ix)[ix>0] - vx(iz,ix+1)[ix+1<N],
-// and written as their DCT-II along z to t.  Grid (ceil(ceil(N/2) / C), B).
-__global__ __launch_bounds__(256) void k_nm_z_fwd(const double *__restrict__ g, const double *__restrict__ bz,
-                                                  const double *__restrict__ bx, const double *__restrict__ dz,
-                                                  const double *__restrict__ dx, double *__restrict__ t,
+// and written as their DCT-II along z to t.  Two elements' ten loads go out together from clamped
+// addresses: 600^2 x 32 (mean over a solve) 93 us, with loads behind branches 171.  Grid (ceil(ceil(N/2) / C), B).  IP: the transform
+// in place (one LDS buffer), else between two.
+template <bool IP>
+__global__ __launch_bounds__(512) void k_nm_z_fwd(const float *__restrict__ g, const double *__restrict__ qz,
+                                                  const double *__restrict__ qx, double *__restrict__ t,
                                                   const int *__restrict__ active, NmArgs A)
 {
     extern __shared__ double2 nm_sm[];
@@ -166,27 +300,45 @@ __global__ __launch_bounds__(256) void k_nm_z_fwd(const double *__restrict__ g, 
     if (!active[b]) return;
     const int N = A.N, C = A.C;
     const size_t o = (size_t)b * N * N;
-    double2 *a0 = nm_sm, *a1 = nm_sm + C * N;
+    double2 *a0 = nm_sm;
     const int col0 = blockIdx.x * 2 * C;
+    const float invN = 1.0f / (float)N;
     auto rhs = [&](int iz, int ix) -> double {
-        if (ix >= N) return 0.0;
-        const size_t k = o + (size_t)ix * N + iz;
+        // clamped addresses and selected values: all loads go out before any is used
+        const int jx = min(ix, N - 1);
+        const size_t k = o + (size_t)jx * N + iz;
+        const double z0 = qz[k], z1 = qz[iz + 1 < N ? k + 1 : k], x0 = qx[k], x1 = qx[jx + 1 < N ? k + N : k];
+        const double gv = (double)g[k];
         double bt = 0.0;
-        if (iz > 0) bt += bz[k] - dz[k];
-        if (iz + 1 < N) bt -= bz[k + 1] - dz[k + 1];
-        if (ix > 0) bt += bx[k] - dx[k];
-        if (ix + 1 < N) bt -= bx[k + N] - dx[k + N];
-        return g[k] - bt;
+        if (iz > 0) bt += z0;
+        if (iz + 1 < N) bt -= z1;
+        if (ix > 0) bt += x0;
+        if (ix + 1 < N) bt -= x1;
+        return ix < N ? gv - bt : 0.0;
     };
-    for (int e = threadIdx.x; e < C * N; e += blockDim.x) {
-        const int c = e / N, i = e - c * N;
-        const int ix = col0 + 2 * c;
-        a0[c * N + nm_perm(i, N)] = make_double2(rhs(i, ix), rhs(i, ix + 1));
+    for (int e0 = threadIdx.x; e0 < C * N; e0 += 2 * blockDim.x) {   // two elements' loads in flight
+        double2 v[2];
+        int at[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int e = min(e0 + h * (int)blockDim.x, C * N - 1);
+            int c, i;
+            divmod_small(e, N, invN, c, i);
+            const int ix = col0 + 2 * c;
+            at[h] = c * N + nm_perm(i, N);
+            v[h] = make_double2(rhs(i, ix), rhs(i, ix + 1));
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            if (e0 + h * (int)blockDim.x < C * N) a0[at[h]] = v[h];
     }
     __syncthreads();
-    const double2 *Z = nm_fft(a0, a1, N, C, A.f, A.tw, false);
+    const double2 *Z = a0;
+    if constexpr (IP) nm_fft_ip(a0, N, C, A.f, A.tw, false);
+    else Z = nm_fft(a0, nm_sm + C * N, N, C, A.f, A.tw, false);
     for (int e = threadIdx.x; e < C * N; e += blockDim.x) {
-        const int c = e / N, k = e - c * N;
+        int c, k;
+        divmod_small(e, N, invN, c, k);
         const int ix = col0 + 2 * c;
         const double2 X = nm_dct_pair(Z + c * N, k, N, A.qw);
         if (ix < N) t[o + (size_t)ix * N + k] = X.x;
@@ -195,54 +347,66 @@ __global__ __launch_bounds__(256) void k_nm_z_fwd(const double *__restrict__ g, 
 }
 
 // Pass 2, along x: rows = pairs of z frequencies (kz, kz + 1); DCT-II along x, divide by
-// 1 + l_kz + l_kx, DCT-III along x, in place in t.
-__global__ __launch_bounds__(256) void k_nm_x(double *__restrict__ t, const int *__restrict__ active, NmArgs A)
+// 1 + l_kz + l_kx, DCT-III along x, in place in t.  The 2 C rows of a workgroup are a
+// 16 C-byte run of every image column: with C = 1 half of every 32 bytes fetched was another
+// workgroup's.  A spectrum point and its mirror image (k, N - k) stay with one thread from the
+// forward to the inverse transform.
+template <bool IP>
+__global__ __launch_bounds__(512) void k_nm_x(double *__restrict__ t, const int *__restrict__ active, NmArgs A)
 {
     extern __shared__ double2 nm_sm[];
     const int b = blockIdx.y;
     if (!active[b]) return;
     const int N = A.N, C = A.C;
     const size_t o = (size_t)b * N * N;
-    double2 *a0 = nm_sm, *a1 = nm_sm + C * N;
+    double2 *a0 = nm_sm;
     const int row0 = blockIdx.x * 2 * C;
     const int R = 2 * C;
+    const float invR = 1.0f / (float)R;
     // element (kz = row0 + r, ix): consecutive threads take consecutive kz
     for (int e = threadIdx.x; e < R * N; e += blockDim.x) {
-        const int ix = e / R, r = e - ix * R;
+        int ix, r;
+        divmod_small(e, R, invR, ix, r);
         const int kz = row0 + r;
         const double v = kz < N ? t[o + (size_t)ix * N + kz] : 0.0;
         reinterpret_cast<double *>(a0 + (r >> 1) * N + nm_perm(ix, N))[r & 1] = v;
     }
     __syncthreads();
-    double2 *Z = nm_fft(a0, a1, N, C, A.f, A.tw, false);
-    double2 *X = Z == a0 ? a1 : a0;
-    for (int e = threadIdx.x; e < C * N; e += blockDim.x) {
-        const int c = e / N, k = e - c * N;
-        const int kz = row0 + 2 * c;
-        double2 v = nm_dct_pair(Z + c * N, k, N, A.qw);
-        const double lk = A.lam[k];
-        v.x /= 1.0 + A.lam[kz < N ? kz : 0] + lk;
-        v.y /= 1.0 + A.lam[kz + 1 < N ? kz + 1 : 0] + lk;
-        X[c * N + k] = v;
+    double2 *Z = a0;
+    if constexpr (IP) nm_fft_ip(a0, N, C, A.f, A.tw, false);
+    else Z = nm_fft(a0, nm_sm + C * N, N, C, A.f, A.tw, false);
+    const int h = N / 2 + 1;
+    const float invh = 1.0f / (float)h;
+    for (int e = threadIdx.x; e < C * h; e += blockDim.x) {
+        int c, k;
+        divmod_small(e, h, invh, c, k);
+        const int kz = row0 + 2 * c, kr = k ? N - k : 0;
+        double2 *Zc = Z + c * N;
+        const double l0 = 1.0 + A.lam[kz < N ? kz : 0], l1 = 1.0 + A.lam[kz + 1 < N ? kz + 1 : 0];
+        double2 v = nm_dct_pair(Zc, k, N, A.qw), vr = nm_dct_pair(Zc, kr, N, A.qw);
+        v.x /= l0 + A.lam[k];
+        v.y /= l1 + A.lam[k];
+        vr.x /= l0 + A.lam[kr];
+        vr.y /= l1 + A.lam[kr];
+        Zc[k] = nm_idct_pair(v, vr, k, N, A.qw);
+        if (kr != k) Zc[kr] = nm_idct_pair(vr, v, kr, N, A.qw);
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < C * N; e += blockDim.x) {
-        const int c = e / N, k = e - c * N;
-        const double2 *Xc = X + c * N;
-        Z[c * N + k] = nm_idct_pair(Xc[k], Xc[k == 0 ? 0 : N - k], k, N, A.qw);
-    }
-    __syncthreads();
-    const double2 *z = nm_fft(Z, X, N, C, A.f, A.tw, true);
+    const double2 *z = Z;
+    if constexpr (IP) nm_fft_ip(a0, N, C, A.f, A.tw, true);
+    else z = nm_fft(Z, Z == a0 ? nm_sm + C * N : a0, N, C, A.f, A.tw, true);
     const double inv = 1.0 / N;
     for (int e = threadIdx.x; e < R * N; e += blockDim.x) {
-        const int ix = e / R, r = e - ix * R;
+        int ix, r;
+        divmod_small(e, R, invR, ix, r);
         const int kz = row0 + r;
         if (kz < N) t[o + (size_t)ix * N + kz] = reinterpret_cast<const double *>(z + (r >> 1) * N + nm_perm(ix, N))[r & 1] * inv;
     }
 }
 
 // Pass 3, along z: rows = pairs of image columns; DCT-III along z from t into u.
-__global__ __launch_bounds__(256) void k_nm_z_inv(const double *__restrict__ t, double *__restrict__ u,
+template <bool IP>
+__global__ __launch_bounds__(512) void k_nm_z_inv(const double *__restrict__ t, double *__restrict__ u,
                                                   const int *__restrict__ active, NmArgs A)
 {
     extern __shared__ double2 nm_sm[];
@@ -250,10 +414,12 @@ __global__ __launch_bounds__(256) void k_nm_z_inv(const double *__restrict__ t, 
     if (!active[b]) return;
     const int N = A.N, C = A.C;
     const size_t o = (size_t)b * N * N;
-    double2 *a0 = nm_sm, *a1 = nm_sm + C * N;
+    double2 *a0 = nm_sm;
     const int col0 = blockIdx.x * 2 * C;
+    const float invN = 1.0f / (float)N;
     for (int e = threadIdx.x; e < C * N; e += blockDim.x) {
-        const int c = e / N, k = e - c * N;
+        int c, k;
+        divmod_small(e, N, invN, c, k);
         const int ix = col0 + 2 * c;
         const int kr = k == 0 ? 0 : N - k;
         double2 xk = make_double2(0.0, 0.0), xr = make_double2(0.0, 0.0);
@@ -262,10 +428,13 @@ __global__ __launch_bounds__(256) void k_nm_z_inv(const double *__restrict__ t, 
         a0[c * N + k] = nm_idct_pair(xk, xr, k, N, A.qw);
     }
     __syncthreads();
-    const double2 *z = nm_fft(a0, a1, N, C, A.f, A.tw, true);
+    const double2 *z = a0;
+    if constexpr (IP) nm_fft_ip(a0, N, C, A.f, A.tw, true);
+    else z = nm_fft(a0, nm_sm + C * N, N, C, A.f, A.tw, true);
     const double inv = 1.0 / N;
     for (int e = threadIdx.x; e < C * N; e += blockDim.x) {
-        const int c = e / N, i = e - c * N;
+        int c, i;
+        divmod_small(e, N, invN, c, i);
         const int ix = col0 + 2 * c;
         const double2 v = z[c * N + nm_perm(i, N)];
         if (ix < N) u[o + (size_t)ix * N + i] = v.x * inv;
@@ -276,7 +445,8 @@ __global__ __launch_bounds__(256) void k_nm_z_inv(const double *__restrict__ t, 
 // SB_ITV2's stop test on the device: an active item stops once
 // ||u_prev - u|| / ||u|| <= 1e-3 (NaN also stops, as MATLAB's while condition); cnt counts
 // the steps in which some item was active
-__global__ void k_tv_active(const double *__restrict__ part, int *__restrict__ active, int B, int *cnt)
+__global__ void k_tv_active(const double *__restrict__ part, int *__restrict__ active, int *__restrict__ take,
+                            int which, int B, int *cnt)
 {
     __shared__ int any;
     if (threadIdx.x == 0) any = 0;
@@ -284,6 +454,7 @@ __global__ void k_tv_active(const double *__restrict__ part, int *__restrict__ a
     for (int b = threadIdx.x; b < B; b += blockDim.x) {
         if (!active[b]) continue;
         any = 1;
+        take[b] = 1 + which;   // the buffer that holds this item's newest image
         double sa = 0.0, sb = 0.0;
         for (int i = 0; i < kRedBlocks; ++i) {
             sa += part[((size_t)Q_A * B + b) * kRedBlocks + i];
@@ -296,11 +467,13 @@ __global__ void k_tv_active(const double *__restrict__ part, int *__restrict__ a
     if (threadIdx.x == 0 && any) cnt[0] += 1;
 }
 
-// Bub = B u + b; s = |Bub|; d = max(s - mu, 0) Bub / s (0 where s == 0); b = Bub - d;
-// ||u_prev - u||^2 -> part Q_A, ||u||^2 -> Q_B; u_prev <- u
-__global__ __launch_bounds__(256) void k_tv_shrink(const double *__restrict__ u, double *__restrict__ up,
+// Bub = B u + b; s = |Bub|; d = max(s - mu, 0) Bub / s (0 where s == 0); b = Bub - d, q = b - d (all
+// that the next right-hand side reads of b and d);
+// ||u_prev - u||^2 -> part Q_A, ||u||^2 -> Q_B.  Bound by memory: eight arrays of the size of the image,
+// 32 x 600^2: 110 us a step, where copying u to u_prev as well and 64-bit divisions took 124.
+__global__ __launch_bounds__(256) void k_tv_shrink(const double *__restrict__ u, const double *__restrict__ up,
                                                    double *__restrict__ bz, double *__restrict__ bx,
-                                                   double *__restrict__ dz, double *__restrict__ dx, int N, int B,
+                                                   double *__restrict__ qz, double *__restrict__ qx, int N, int B,
                                                    const double *__restrict__ mu, const int *__restrict__ active,
                                                    double *part)
 {
@@ -310,7 +483,7 @@ __global__ __launch_bounds__(256) void k_tv_shrink(const double *__restrict__ u,
     if (active[b]) {
         const double m = mu[b];
         for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < P; i += (size_t)gridDim.x * blockDim.x) {
-            const int ix = (int)(i / N), iz = (int)(i - (size_t)ix * N);
+            const int ix = (int)((unsigned)i / (unsigned)N), iz = (int)i - ix * N;   // at most 2048^2 pixels
             const double ui = u[o + i];
             const double gz = iz > 0 ? ui - u[o + i - 1] : 0.0;
             const double gx = ix > 0 ? ui - u[o + i - N] : 0.0;
@@ -318,14 +491,14 @@ __global__ __launch_bounds__(256) void k_tv_shrink(const double *__restrict__ u,
             const double s = sqrt(az * az + ax * ax);
             const double f = s > 0.0 ? fmax(s - m, 0.0) / s : 0.0;
             const double nz = f * az, nx = f * ax;
-            dz[o + i] = nz;
-            dx[o + i] = nx;
-            bz[o + i] = az - nz;
-            bx[o + i] = ax - nx;
+            const double rz = az - nz, rx = ax - nx;
+            bz[o + i] = rz;
+            bx[o + i] = rx;
+            qz[o + i] = rz - nz;
+            qx[o + i] = rx - nx;
             const double df = up[o + i] - ui;
             e += df * df;
             nu += ui * ui;
-            up[o + i] = ui;
         }
     }
     block_sum_store(e, part, Q_A, b, B);
@@ -334,10 +507,16 @@ __global__ __launch_bounds__(256) void k_tv_shrink(const double *__restrict__ u,
 
 __global__ void k_tv_zero_cnt(int *cnt) { cnt[0] = 0; }
 
-__global__ void k_tv_store(const double *__restrict__ u, float *__restrict__ x, size_t n)
+// x = (float) u for the items with take[b]
+__global__ void k_tv_store(const double *__restrict__ u0, const double *__restrict__ u1, float *__restrict__ x,
+                           const int *__restrict__ take, size_t P)
 {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        x[i] = (float)u[i];
+    const int t = take[blockIdx.y];
+    if (!t) return;
+    const double *u = t == 1 ? u0 : u1;
+    const size_t o = (size_t)blockIdx.y * P;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < P; i += (size_t)gridDim.x * blockDim.x)
+        x[o + i] = (float)u[o + i];
 }
 
 // isotropic TV with MATLAB gradient (central differences inside, one-sided at edges) -> Q_C
@@ -485,13 +664,15 @@ __global__ void k_tv_nnls(const float *__restrict__ x, float *__restrict__ w, fl
     }
 }
 
-struct TvWork {
+struct TvWork {   // stream-ordered scratch
+    hipStream_t s;
     std::vector<void *> all;
-    ~TvWork() { for (void *p : all) (void)hipFree(p); }
+    explicit TvWork(hipStream_t st) : s(st) {}
+    ~TvWork() { for (void *p : all) (void)hipFreeAsync(p, s); }
     template <typename T>
     int alloc(T **p, size_t n)
     {
-        hipError_t e = hipMalloc((void **)p, (n ? n : 1) * sizeof(T));
+        hipError_t e = scratch_malloc((void **)p, (n ? n : 1) * sizeof(T), s);
         if (e != hipSuccess) {
             (void)hipGetLastError();
             return set_error(MBREC_ERR_HIP, "mbrec:alloc", "TV workspace allocation failed");
@@ -508,9 +689,10 @@ struct TvProx {
     double2 *tw = nullptr, *qw = nullptr;          // e^{-2 pi i j/N}, e^{-i pi k/2N}
     double *lam = nullptr;                         // 4 sin^2(pi k / 2N)
     NmArgs nm{};
-    double *g = nullptr, *u = nullptr, *up = nullptr, *bz = nullptr, *bx = nullptr, *dz = nullptr, *dx = nullptr;
+    double *u[2] = {nullptr, nullptr}, *bz = nullptr, *bx = nullptr, *qz = nullptr, *qx = nullptr;
     double *t1 = nullptr, *mu = nullptr, *part = nullptr, *sums = nullptr;
-    int *active = nullptr, *cnt = nullptr;
+    int *active = nullptr, *take = nullptr, *cnt = nullptr;
+    bool ip = false;                               // in-place transforms (N a product of 2, 3, 5 and 7)
 };
 
 // N's prime factors, radix 4 first (fewer stages), then 2, 3, 5, 7, ...
@@ -532,6 +714,21 @@ static bool nm_factors(int N, NmFactors &f)
     return true;
 }
 
+// factors for the in-place transform: odd ones first (the first stages' LDS writes then fall on
+// different banks), then 8, 4, 2; false where another prime remains
+static bool nm_factors_ip(int N, NmFactors &f)
+{
+    f.n = 0;
+    int n = N, e2 = 0;
+    for (int p : {5, 3, 7})
+        for (; n % p == 0; n /= p) f.p[f.n++] = p;
+    for (; n % 2 == 0; n /= 2) ++e2;
+    for (; e2 >= 3 && e2 != 4; e2 -= 3) f.p[f.n++] = 8;
+    for (; e2 >= 2; e2 -= 2) f.p[f.n++] = 4;
+    if (e2) f.p[f.n++] = 2;
+    return n == 1;
+}
+
 static int prox_setup(TvProx &T, TvWork &w, int N, int B, hipStream_t s)
 {
     if (N > kNmMaxN)
@@ -540,12 +737,13 @@ static int prox_setup(TvProx &T, TvWork &w, int N, int B, hipStream_t s)
     T.B = B;
     const size_t P = (size_t)N * N, n = P * B;
     int rc;
-    double **bufs[] = {&T.g, &T.u, &T.up, &T.bz, &T.bx, &T.dz, &T.dx, &T.t1};
+    double **bufs[] = {&T.u[0], &T.u[1], &T.bz, &T.bx, &T.qz, &T.qx, &T.t1};
     for (double **b : bufs)
         if ((rc = w.alloc(b, n))) return rc;
     if ((rc = w.alloc(&T.tw, N)) || (rc = w.alloc(&T.qw, N)) || (rc = w.alloc(&T.lam, N)) ||
         (rc = w.alloc(&T.mu, B)) || (rc = w.alloc(&T.part, (size_t)kMaxQ * B * kRedBlocks)) ||
-        (rc = w.alloc(&T.sums, 6 * (size_t)B)) || (rc = w.alloc(&T.active, B)) || (rc = w.alloc(&T.cnt, 1)))
+        (rc = w.alloc(&T.sums, 6 * (size_t)B)) || (rc = w.alloc(&T.active, B)) || (rc = w.alloc(&T.take, B)) ||
+        (rc = w.alloc(&T.cnt, 1)))
         return rc;
     std::vector<double2> tw(N), qw(N);
     std::vector<double> lam(N);
@@ -559,11 +757,15 @@ static int prox_setup(TvProx &T, TvWork &w, int N, int B, hipStream_t s)
     MBREC_HIP(hipMemcpyAsync(T.lam, lam.data(), sizeof(double) * N, hipMemcpyHostToDevice, s));
     MBREC_HIP(hipStreamSynchronize(s));
     T.nm.N = N;
-    // row pairs per workgroup: about 512 complex points (at 600^2 one pair, 19 KB of LDS,
-    // eight workgroups per CU; measured 0.58 ms per Neumann solve of 32 images against
-    // 1.00 ms with three pairs, 57.6 KB and two workgroups per CU)
-    T.nm.C = std::max(1, std::min(4, 512 / N));
-    if (!nm_factors(N, T.nm.f))
+    // row pairs per workgroup: in place up to eight, as many as 4096 complex points hold (64 KB of LDS,
+    // two workgroups of 512 per CU; at 600^2 six, 96-byte runs in pass 2); else about 512 points
+    // between two buffers
+    T.ip = nm_factors_ip(N, T.nm.f);
+    if (T.ip)
+        T.nm.C = std::max(1, std::min({8, kNmIpPoints / N, (N + 1) / 2}));
+    else
+        T.nm.C = std::max(1, std::min(4, 512 / N));
+    if (!T.ip && !nm_factors(N, T.nm.f))
         return set_error(MBREC_ERR_ARG, "mbrec:tvSize", "rec_nn_with_TV_reg: too many prime factors in the image side");
     T.nm.tw = T.tw;
     T.nm.qw = T.qw;
@@ -571,25 +773,35 @@ static int prox_setup(TvProx &T, TvWork &w, int N, int B, hipStream_t s)
     return MBREC_OK;
 }
 
-// u = (I + B'B)^-1 (g - B'(b - d)) for every active item: DCT-II along z (rhs formed on
+// u = (I + B'B)^-1 (g - B'(b - d)) for every active item (g: the prox's FP32 input): DCT-II along z (rhs formed on
 // load), along x (forward, divide by 1 + l_kz + l_kx, inverse), DCT-III along z
-static void neumann_solve(TvProx &T, hipStream_t s)
+static void neumann_solve(TvProx &T, const float *g, double *u, hipStream_t s)
 {
     const int N = T.N, C = T.nm.C;
     const dim3 grid((unsigned)(((N + 1) / 2 + C - 1) / C), (unsigned)T.B);
+    if (T.ip) {
+        const dim3 block(C * N > 2048 ? 512 : 256);
+        const size_t lds = sizeof(double2) * C * N;
+        hipLaunchKernelGGL(k_nm_z_fwd<true>, grid, block, lds, s, g, (const double *)T.qz, (const double *)T.qx, T.t1,
+                           (const int *)T.active, T.nm);
+        hipLaunchKernelGGL(k_nm_x<true>, grid, block, lds, s, T.t1, (const int *)T.active, T.nm);
+        hipLaunchKernelGGL(k_nm_z_inv<true>, grid, block, lds, s, (const double *)T.t1, u, (const int *)T.active, T.nm);
+        return;
+    }
     const size_t lds = sizeof(double2) * 2 * C * N;
-    hipLaunchKernelGGL(k_nm_z_fwd, grid, dim3(256), lds, s, (const double *)T.g, (const double *)T.bz,
-                       (const double *)T.bx, (const double *)T.dz, (const double *)T.dx, T.t1,
+    hipLaunchKernelGGL(k_nm_z_fwd<false>, grid, dim3(256), lds, s, g, (const double *)T.qz, (const double *)T.qx, T.t1,
                        (const int *)T.active, T.nm);
-    hipLaunchKernelGGL(k_nm_x, grid, dim3(256), lds, s, T.t1, (const int *)T.active, T.nm);
-    hipLaunchKernelGGL(k_nm_z_inv, grid, dim3(256), lds, s, (const double *)T.t1, T.u, (const int *)T.active, T.nm);
+    hipLaunchKernelGGL(k_nm_x<false>, grid, dim3(256), lds, s, T.t1, (const int *)T.active, T.nm);
+    hipLaunchKernelGGL(k_nm_z_inv<false>, grid, dim3(256), lds, s, (const double *)T.t1, u, (const int *)T.active, T.nm);
 }
 
 // x (FP32, [B][N][N]) <- SB_ITV2(z, mu_b) per item; mu host [B]; items with skip[b] are left as they are.
 // The stop test runs on the device after every split-Bregman step; the host reads the
 // active flags every kTvCheck steps (an item that stopped inside a group is not updated
-// again, so the result is the per-step loop's).
+// again, so the result is the per-step loop's).  The image alternates between two buffers from
+// step to step (shrink reads both and writes neither); take[b] names the one an item ended in.
 constexpr int kTvCheck = 4;
+static_assert(kTvCheck % 2 == 0, "the step after a group writes the buffer the group's first step wrote");
 
 static int tv_prox(TvProx &T, const float *z, float *x, const std::vector<double> &mu,
                    const std::vector<int> &skip, hipStream_t s, int *iters_out)
@@ -600,25 +812,28 @@ static int tv_prox(TvProx &T, const float *z, float *x, const std::vector<double
     for (int b = 0; b < B; ++b) act[b] = skip[b] ? 0 : 1;
     MBREC_HIP(hipMemcpyAsync(T.mu, mu.data(), sizeof(double) * B, hipMemcpyHostToDevice, s));
     MBREC_HIP(hipMemcpyAsync(T.active, act.data(), sizeof(int) * B, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_tv_load, dim3(nblk(n)), dim3(256), 0, s, z, T.g, T.up, T.bz, T.bx, T.dz, T.dx, n);
+    MBREC_HIP(hipMemcpyAsync(T.take, act.data(), sizeof(int) * B, hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_tv_load, dim3(nblk(n)), dim3(256), 0, s, z, T.u[1], T.bz, T.bx, T.qz, T.qx, n);
     hipLaunchKernelGGL(k_tv_zero_cnt, dim3(1), dim3(1), 0, s, T.cnt);
     for (;;) {
         bool any = false;
         for (int b = 0; b < B; ++b) any = any || act[b];
         if (!any) break;
         for (int c = 0; c < kTvCheck; ++c) {
-            neumann_solve(T, s);
-            hipLaunchKernelGGL(k_tv_shrink, vgrid(B), dim3(256), 0, s, (const double *)T.u, T.up, T.bz, T.bx, T.dz,
-                               T.dx, N, B, (const double *)T.mu, (const int *)T.active, T.part);
-            hipLaunchKernelGGL(k_tv_active, dim3(1), dim3(256), 0, s, (const double *)T.part, T.active, B, T.cnt);
+            double *u = T.u[c & 1];
+            neumann_solve(T, z, u, s);
+            hipLaunchKernelGGL(k_tv_shrink, vgrid(B), dim3(256), 0, s, (const double *)u,
+                               (const double *)T.u[(c & 1) ^ 1], T.bz, T.bx, T.qz, T.qx, N, B, (const double *)T.mu,
+                               (const int *)T.active, T.part);
+            hipLaunchKernelGGL(k_tv_active, dim3(1), dim3(256), 0, s, (const double *)T.part, T.active, T.take, c & 1,
+                               B, T.cnt);
         }
         MBREC_HIP(hipMemcpyAsync(act.data(), T.active, sizeof(int) * B, hipMemcpyDeviceToHost, s));
         MBREC_HIP(hipStreamSynchronize(s));
     }
     // write back items that were processed
-    for (int b = 0; b < B; ++b)
-        if (!skip[b])
-            hipLaunchKernelGGL(k_tv_store, dim3(nblk(P)), dim3(256), 0, s, (const double *)(T.up + b * P), x + b * P, P);
+    hipLaunchKernelGGL(k_tv_store, dim3(std::min(nblk(P), 256), B), dim3(256), 0, s, (const double *)T.u[0],
+                       (const double *)T.u[1], x, (const int *)T.take, P);
     if (iters_out) {
         MBREC_HIP(hipMemcpyAsync(iters_out, T.cnt, sizeof(int), hipMemcpyDeviceToHost, s));
         MBREC_HIP(hipStreamSynchronize(s));
@@ -635,7 +850,7 @@ int nnls_tv(Plan *p, const float *y, int B, int coupled, int num_iter, double ta
     const int N = p->Nz;
     const size_t np = (size_t)p->P, ns = (size_t)p->D * p->nT;
     const int G = coupled ? 1 : B;
-    TvWork w;
+    TvWork w(s);
     TvProx T;
     int rc;
     float *x, *px, *z, *dxv, *v, *rc_, *atr, *rs, *ts;
@@ -769,9 +984,9 @@ extern "C" int mbrec_sb_itv2_dev(const float *g, int N, int B, const double *mu,
 {
     if (!g || !u || !mu || N <= 0 || B <= 0)
         return set_error(MBREC_ERR_ARG, "mbrec:args", "SB_ITV2: invalid arguments");
-    TvWork w;
-    TvProx T;
     const hipStream_t st = (hipStream_t)s;
+    TvWork w(st);
+    TvProx T;
     int rc;
     if ((rc = prox_setup(T, w, N, B, st))) return rc;
     std::vector<double> m(mu, mu + B);

@@ -214,3 +214,27 @@ def test_sb_itv2_device_matches_oracle(require_gpu, N, mu):
         its.append(k)
         assert rel_l2(u[b].ravel(), ref) < 1e-6, b
     assert it == max(its)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [1, 2, 3, 5, 16, 26, 35, 42, 210, 506, 512, 720, 1025, 1536, 2048])
+def test_sb_itv2_transform_sizes(require_gpu, N):
+    """Every butterfly of the in-place transform (2, 3, 4, 5, 7, 8), sides with another prime (26,
+    506, 1025), the smallest and the largest side, 8, 4, 2 and 1 row pairs per workgroup with a
+    remainder; images that stop after different steps (their results lie in different buffers).
+    FP32 output of an FP64 iteration that stops on the oracle's step: 2^-24 relative rounding, with
+    the existing comparison's limit of 1e-6."""
+    from mbrec.solvers import SB_ITV2
+    print(f"sb_itv2 transform N={N}", flush=True)
+    mus = np.array([0.2, 0.02, 1.5]) if N <= 720 else np.array([0.05])
+    g = rng(N).standard_normal((len(mus), N, N)).astype(np.float32)
+    g += 2.0 * (np.arange(N) > N / 3)
+    g = g.astype(np.float32)
+    u, it = SB_ITV2(g, mus)
+    B = O.diff_oper(N)
+    its = []
+    for b in range(len(mus)):
+        ref, k = O.sb_itv2(g[b].astype(np.float64).ravel(), mus[b], B, exact=True)
+        its.append(k)
+        assert rel_l2(u[b].ravel(), ref) < 1e-6, b
+    assert it == max(its)
