@@ -586,17 +586,20 @@ __host__ __device__ constexpr int fir16_window(int Lp) { return 16 * fir16_nblk(
 
 // LPT > 0: the padded tap count Lp known at compile time (the tap loop unrolls fully, the
 // register window needs no moves and the LDS offsets are immediates); LPT = 0: any L.
-// SPLIT: for few rows (one sinogram: 256 tiles for the whole filter) both halves of the
-// workgroup take the same tile, half 0 the first ceil(Lp / 32) groups of 16 taps and half
-// 1 the rest, and the two FP64 partial sums are added at the end (one tile per workgroup,
-// twice the workgroups; the sum of each half in tap order, then the two halves).
-template <int LPT, bool SPLIT = false>
-__global__ __launch_bounds__(256) void k_fir16(const float *__restrict__ x, float *__restrict__ out,
+// PARTS > 1: for few rows (one sinogram: 256 tiles for the whole filter, one workgroup per CU)
+// PARTS groups of 128 threads take the same tile, each a run of the groups of 16 taps, and the
+// FP64 partial sums are added at the end (the sum of each part in tap order, then the parts).
+// With two parts every SIMD holds one wave, which waits for its own taps and window rows; with
+// four a second wave works meanwhile, and each part adds a quarter of the outputs: 11.8 -> 9.3 us
+// for 256 rows of 2030 samples (the 201-tap IR; other lengths keep two parts, their LDS).
+template <int LPT, int PARTS = 1>
+__global__ __launch_bounds__(PARTS > 1 ? 128 * PARTS : 256) void k_fir16(const float *__restrict__ x, float *__restrict__ out,
                                                const double *__restrict__ taps64, int L, int per_det, int off, int D,
                                                int nT, int rows, float scale, const int2 *__restrict__ win)
 {
     extern __shared__ float sm[];
     const int Lp = LPT ? LPT : fir16_padded_taps(L), nx = fir16_window(Lp), NBLK = fir16_nblk(Lp);
+    constexpr bool SPLIT = PARTS > 1;
     const int hf = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7), lt = threadIdx.x & 127;
     float *xs = SPLIT ? sm : sm + (size_t)hf * nx;
     const int ntile = (nT + kFirSpan - 1) / kFirSpan;
@@ -619,7 +622,7 @@ __global__ __launch_bounds__(256) void k_fir16(const float *__restrict__ x, floa
     };
     auto stx = [&](int i, float v) { xs[(i & 15) * NBLK + (i >> 4)] = v; };
     if constexpr (SPLIT)
-        stage_batched<8, 256>((int)threadIdx.x, nx, ldx, stx);
+        stage_batched<16 / PARTS, 128 * PARTS>((int)threadIdx.x, nx, ldx, stx);
     else
         stage_batched<8, 128>(lt, nx, ldx, stx);
     // the row's taps, FP64 and zero-padded to Lp, read as scalars (uniform per wave)
@@ -634,8 +637,8 @@ __global__ __launch_bounds__(256) void k_fir16(const float *__restrict__ x, floa
     // tap groups [i0a, i0b) of this thread (all of them unless SPLIT); the register window
     // at the start of the group at i0 is W[w] = element (w + 8, blk - i0 / 16) for w < 8 and
     // (w - 8, blk - i0 / 16 + 1) for w >= 8 (the state the shifts below leave)
-    const int Sp = 16 * ((Lp / 16 + 1) / 2);
-    const int i0a = SPLIT && hf ? Sp : 0;
+    auto first = [](int lp, int h) { return 16 * (lp / 16 * h / PARTS); };
+    const int i0a = SPLIT ? first(Lp, hf) : 0;
     double W[23], acc[kFirOut];
 #pragma unroll
     for (int w = 0; w < 8; ++w) W[w] = (double)xs[(w + 8) * NBLK + blk - i0a / 16];
@@ -664,16 +667,17 @@ __global__ __launch_bounds__(256) void k_fir16(const float *__restrict__ x, floa
         if (i0 + 16 < Lp) shift(blk - i0 / 16 - 1, 8);
     };
     if constexpr (SPLIT && LPT > 0) {
-        constexpr int S = 16 * ((LPT / 16 + 1) / 2);
-        if (hf == 0) {
+        auto part = [&](auto h) {
+            constexpr int H = decltype(h)::value, S0 = 16 * (LPT / 16 * H / PARTS), S1 = 16 * (LPT / 16 * (H + 1) / PARTS);
 #pragma unroll
-            for (int i0 = 0; i0 < S; i0 += 16) step(i0);
-        } else {
-#pragma unroll
-            for (int i0 = S; i0 < LPT; i0 += 16) step(i0);
-        }
+            for (int i0 = S0; i0 < S1; i0 += 16) step(i0);
+        };
+        if (hf == 0) part(std::integral_constant<int, 0>{});
+        else if (PARTS == 2 || hf == 1) part(std::integral_constant<int, 1>{});
+        else if (hf == 2) part(std::integral_constant<int, 2>{});
+        else part(std::integral_constant<int, 3>{});
     } else if constexpr (SPLIT) {
-        for (int i0 = i0a; i0 < (hf ? Lp : Sp); i0 += 16) step(i0);
+        for (int i0 = i0a; i0 < first(Lp, hf + 1); i0 += 16) step(i0);
     } else if constexpr (LPT > 0) {
 #pragma unroll
         for (int i0 = 0; i0 < LPT; i0 += 16) step(i0);
@@ -681,24 +685,24 @@ __global__ __launch_bounds__(256) void k_fir16(const float *__restrict__ x, floa
         for (int i0 = 0; i0 < Lp; i0 += 16) step(i0);   // Lp is a multiple of 16
     }
     __syncthreads();   // xs is reused for the outputs (same layout)
-    if constexpr (SPLIT) {   // half 1's partial sums through LDS (past xs) into half 0's
+    if constexpr (SPLIT) {   // the parts' partial sums through LDS (past xs); part h then adds its outputs' sums
         double *ex = reinterpret_cast<double *>(sm + nx);
-        if (hf) {
+        constexpr int KP = kFirOut / PARTS;
 #pragma unroll
-            for (int k = 0; k < kFirOut; ++k) ex[k * 128 + lt] = acc[k];
-        }
+        for (int k = 0; k < kFirOut; ++k) ex[(hf * kFirOut + k) * 128 + lt] = acc[k];
         __syncthreads();
-        if (!hf) {
 #pragma unroll
-            for (int k = 0; k < kFirOut; ++k) {
-                const int t = t0 + 16 * lt + k;
-                xs[k * NBLK + lt] = (t >= lo && t < hi) ? scale * (float)(acc[k] + ex[k * 128 + lt]) : 0.0f;
-            }
+        for (int j = 0; j < KP; ++j) {
+            const int k = hf * KP + j, t = t0 + 16 * lt + k;
+            double v = ex[k * 128 + lt];
+#pragma unroll
+            for (int h = 1; h < PARTS; ++h) v += ex[(h * kFirOut + k) * 128 + lt];
+            xs[k * NBLK + lt] = (t >= lo && t < hi) ? scale * (float)v : 0.0f;
         }
         __syncthreads();
         if (!live) return;
         float *orow = out + (size_t)row * nT;
-        for (int i = threadIdx.x; i < kFirSpan && t0 + i < nT; i += 256) orow[t0 + i] = xs[(i & 15) * NBLK + (i >> 4)];
+        for (int i = threadIdx.x; i < kFirSpan && t0 + i < nT; i += 128 * PARTS) orow[t0 + i] = xs[(i & 15) * NBLK + (i >> 4)];
         return;
     }
 #pragma unroll
@@ -4042,15 +4046,16 @@ static int launch_fir(Plan *p, const float *x, float *out, int B, bool corr, flo
     if (lds16 <= kLdsBudget && p->d_ir64) {
         const int rows = B * p->D, ntile = (p->nT + kFirSpan - 1) / kFirSpan;
         const size_t nblk = ((size_t)rows * ntile + 1) / 2;
-        // few tiles (fewer than two per CU): one tile per workgroup, the taps split between its halves
-        const size_t ldsp = sizeof(float) * (size_t)fir16_window(Lp) + sizeof(double) * 128 * kFirOut;
+        // few tiles (fewer than two per CU): one tile per workgroup, the taps split between its parts
+        const int parts = Lp == 208 ? 4 : 2;
+        const size_t ldsp = sizeof(float) * (size_t)fir16_window(Lp) + sizeof(double) * 128 * kFirOut * parts;
         if ((size_t)rows * ntile < 512 && ldsp <= kLdsBudget) {
             const dim3 gp((unsigned)((size_t)rows * ntile));
             if (Lp == 208)
-                hipLaunchKernelGGL((k_fir16<208, true>), gp, dim3(256), ldsp, s, x, out, corr ? p->d_irf64 : p->d_ir64,
+                hipLaunchKernelGGL((k_fir16<208, 4>), gp, dim3(512), ldsp, s, x, out, corr ? p->d_irf64 : p->d_ir64,
                                    L, p->ir_per_det, off, p->D, p->nT, rows, scale, win);
             else
-                hipLaunchKernelGGL((k_fir16<0, true>), gp, dim3(256), ldsp, s, x, out, corr ? p->d_irf64 : p->d_ir64,
+                hipLaunchKernelGGL((k_fir16<0, 2>), gp, dim3(256), ldsp, s, x, out, corr ? p->d_irf64 : p->d_ir64,
                                    L, p->ir_per_det, off, p->D, p->nT, rows, scale, win);
             MBREC_HIP(hipGetLastError());
             return MBREC_OK;

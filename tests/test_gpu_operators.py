@@ -467,6 +467,29 @@ def test_model_operators_generic_ir_length(per_det):
     assert rel_l2(xt.reshape(2, -1), orc.transpose(s).reshape(2, -1)) < TOL_OP
 
 
+@pytest.mark.parametrize("L,nT,D,B", [(1, 40, 3, 1), (15, 300, 5, 1), (33, 2053, 5, 1), (193, 190, 3, 2),
+                                      (201, 2048, 7, 1), (207, 2053, 5, 3), (201, 300, 257, 2)])
+def test_ir_filter_tap_split(L, nT, D, B):
+    """The IR filter with its taps split over the parts of a workgroup (few rows): four parts for
+    193..208 taps, two else, one group of taps only, records shorter than the taps, one and two
+    tiles per record with a remainder; and the unsplit form above 511 tiles.  FP64 sums of FP32
+    samples: the other operator tests' limit."""
+    import torch
+    from mbrec.model import DevicePlan
+    _log(f"IR filter split L={L} nT={nT} D={D} B={B}")
+    Nz, Nx, R = 12, 10, 2.6666666666666665
+    tt = random_tt(Nz * Nx, D, nT, R, seed=L + nT, spill=0.05)
+    ir = rng(L).standard_normal(L)
+    plan = DevicePlan(Nz, Nx, D, nT, R, tt.T, ir=ir)
+    orc = O.Model(Nz, Nx, np.ascontiguousarray(tt.T), nT, R, ir=ir)
+    x = rng(95).uniform(0, 1, (B, Nx, Nz))
+    y = plan.forward(torch.tensor(x, dtype=torch.float32).cuda()).cpu().numpy()
+    assert rel_l2(y.reshape(B, -1), orc.forward(x).reshape(B, -1)) < TOL_OP
+    s = rng(96).standard_normal((B, D, nT))
+    xt = plan.transpose(torch.tensor(s, dtype=torch.float32).cuda()).cpu().numpy()
+    assert rel_l2(xt.reshape(B, -1), orc.transpose(s).reshape(B, -1)) < TOL_OP
+
+
 @pytest.mark.parametrize("fir_mfma", [True, False])
 @pytest.mark.parametrize("sir", [False, True])
 def test_model_operators_match_oracle(sir, fir_mfma):
