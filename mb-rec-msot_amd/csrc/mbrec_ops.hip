@@ -3279,8 +3279,8 @@ static void scatter_bl(Plan *p, const float *imgI, int B, int Bp, hipStream_t s)
 // batch-lane kernel with lane groups of -value sinograms
 // SIR forward in pull form (records of build_sir_pull): scatter choices of their own, the
 // bins written directly (no bucket windows).  kSirPull: for one sinogram the band form on the
-// vector ALUs (windows of more than 31 taps: the lane-group kernel; the default there), else the batch-lane kernel with 24 samples and 2 records in
-// flight per wave; kSirPull + 1 .. 3: batch-lane kernels with (16 samples, 4 records),
+// vector ALUs, the default there (windows of more than 31 taps: the lane-group kernel), else the
+// batch-lane kernel with 24 samples and 2 records in flight per wave; kSirPull + 1 .. 3: batch-lane kernels with (16 samples, 4 records),
 // (16, 2), (32, 1); kSirBand (batches; the default there): every record visited once by
 // the wave of its first-sample band, the overlapping wave rows summed in a second pass
 constexpr int kSirPull = 1000, kSirPullVariants = 5, kSirBand = kSirPull + 4;

@@ -15,7 +15,7 @@
 // Numerics: activations and activation gradients are stored in bfloat16
 // (round to nearest even) in pixel-major / channel-minor order; every 3x3
 // convolution with >= 32 input channels runs on the matrix cores
-// (v_mfma_f32_16x16x32_bf16, FP32 accumulation) as an implicit GEMM over
+// (v_mfma_f32_32x32x16_bf16, FP32 accumulation) as an implicit GEMM over
 // (pixels x output channels x 9*input channels); its input gradient is the same
 // kernel with the flipped, transposed filter, and its filter gradient an
 // implicit GEMM over pixels.  The first convolution (one input channel), the
