@@ -420,7 +420,7 @@ int mbrec_unet_train_step(mbrec_unet net, const float *in, const float *target, 
                           float beta1, float beta2, float eps, double *loss_host, mbrec_stream s);
 /* One 3x3 zero-padded convolution on the matrix cores: x bf16 [N][H][W][Cin],
  * w bf16 [Cout][3][3][Cin], y bf16 [N][H][W][Cout]; relu=1: y = relu(conv + bias),
- * relu=0: y = conv (bias must be NULL).  Cin, Cout multiples of 32. */
+ * relu=0: y = conv (bias must be NULL).  Cin, Cout multiples of 32, N H W below 2^30 - 64. */
 int mbrec_conv3x3_bf16(const uint16_t *x, const uint16_t *w, const float *bias, uint16_t *y, int N, int H, int W,
                        int Cin, int Cout, int relu, mbrec_stream s);
 

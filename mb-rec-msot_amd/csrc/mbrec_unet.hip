@@ -25,6 +25,7 @@
 
 #include <cmath>
 #include <algorithm>
+#include <type_traits>
 
 namespace mbrec {
 
@@ -111,7 +112,7 @@ struct ConvArgs {
     int n_low;
     const float *hw, *hb, *s;
     float *on, *out;
-    int N, H, W, Wp, tiles_x, ntiles, ncot;
+    int N, H, W, Wp, tiles_x, ntiles, ncot, tile0;
 };
 
 // memory -> LDS, 16 bytes per lane; dst is the wave's base
@@ -121,24 +122,26 @@ __device__ __forceinline__ void copy_to_lds(const uint16_t *src, uint16_t *dst)
                                      (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
 }
 
-// 16-byte slot `slot` (8 channels) of virtual column X, row h: its index from c.p + c.co, or -1 outside the images
-__device__ __forceinline__ int conv_slot(const ConvSrc &c, int X, int h, int slot, int N, int H, int W, int Wp)
+// 16-byte slot `slot` (8 channels) of virtual column X, row h: its index from c.p + c.co, or -1 outside the
+// images (T: int below 2^31 slots, 32 GB of input, else 64 bits)
+template <typename T = int>
+__device__ __forceinline__ T conv_slot(const ConvSrc &c, int X, int h, int slot, int N, int H, int W, int Wp)
 {
     if (X < 0 || h < 0 || h >= H) return -1;
     const int n = X / Wp, w = X - n * Wp;
     if (n >= N || w >= W) return -1;
     const int px = c.up ? (n * (H / 2) + h / 2) * (W / 2) + w / 2 : (n * H + h) * W + w;
-    return px * (c.cs / 8) + slot;
+    return (T)px * (c.cs / 8) + slot;
 }
 
-template <int NB, int EPI>
+template <int NB, int EPI, typename T = int>
 __global__ __launch_bounds__(256, 2) void k_conv3(const ConvArgs a)
 {
     constexpr int CO = 32 * NB;
     __shared__ __attribute__((aligned(16))) uint16_t s_in[kCvInIt * 256 * 8];
     __shared__ __attribute__((aligned(16))) uint16_t s_w[9 * CO * 32];
     // blocks of one XCD (every eighth) take the channel tiles of a pixel tile in a row
-    const int k = blockIdx.x >> 3, ct = k % a.ncot, sp = (k / a.ncot) * 8 + (blockIdx.x & 7);
+    const int k = blockIdx.x >> 3, ct = k % a.ncot, sp = a.tile0 + (k / a.ncot) * 8 + (blockIdx.x & 7);
     if (sp >= a.ntiles) return;   // whole workgroup, before any barrier
     const int ty = sp / a.tiles_x, tx = sp - ty * a.tiles_x;
     const int X0 = tx * kCvCols, h0 = ty * kCvRows, co0 = ct * CO;
@@ -168,11 +171,11 @@ __global__ __launch_bounds__(256, 2) void k_conv3(const ConvArgs a)
     for (int sidx = 0; sidx < 2; ++sidx) {
         const int nch = sidx ? Cin - a.split : a.split;
         if (nch <= 0) continue;
-        int slot[kCvInIt];
+        T slot[kCvInIt];
 #pragma unroll
         for (int it = 0; it < kCvInIt; ++it) {
             const int e = it * 256 + tid, px = e >> 2, row = px / (kCvCols + 2), col = px - row * (kCvCols + 2);
-            slot[it] = e < kCvIn ? conv_slot(a.src[sidx], X0 + col - 1, h0 + row - 1, (e & 3) ^ ((col >> 1) & 3), a.N, H, W,
+            slot[it] = e < kCvIn ? conv_slot<T>(a.src[sidx], X0 + col - 1, h0 + row - 1, (e & 3) ^ ((col >> 1) & 3), a.N, H, W,
                                              a.Wp)
                                  : -1;
         }
@@ -181,7 +184,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3(const ConvArgs a)
             __syncthreads();   // the previous chunk is no longer read
 #pragma unroll
             for (int it = 0; it < kCvInIt; ++it)
-                copy_to_lds(slot[it] >= 0 ? base + c0 + (size_t)(unsigned)slot[it] * 8 : g_zero_slot,
+                copy_to_lds(slot[it] >= 0 ? base + c0 + (size_t)(std::make_unsigned_t<T>)slot[it] * 8 : g_zero_slot,
                             s_in + (it * 256 + wv * 64) * 8);
 #pragma unroll
             for (int it = 0; it < (9 * CO * 4 + 255) / 256; ++it)
@@ -888,16 +891,20 @@ static ConvArgs conv_args(const ConvSrc &x, int cin, const uint16_t *w, int cout
 }
 
 // 64 output channels per workgroup where they divide (half the input reads per product), else 32
-template <int EPI>
+template <int EPI, typename T = int>
 static void conv_launch(ConvArgs &a, hipStream_t s)
 {
     const bool wide = a.Cout % 64 == 0;
     a.ncot = a.Cout / (wide ? 64 : 32);
-    const dim3 grid((unsigned)((a.ntiles + 7) / 8 * 8 * (size_t)a.ncot));
-    if (wide)
-        hipLaunchKernelGGL((k_conv3<2, EPI>), grid, dim3(256), 0, s, a);
-    else
-        hipLaunchKernelGGL((k_conv3<1, EPI>), grid, dim3(256), 0, s, a);
+    // a launch holds fewer than 2^32 threads: 2^23 workgroups at most, in whole runs of eight tiles
+    const int run = std::max(8, (1 << 23) / a.ncot / 8 * 8);
+    for (a.tile0 = 0; a.tile0 < a.ntiles; a.tile0 += run) {
+        const dim3 grid((unsigned)((std::min(run, a.ntiles - a.tile0) + 7) / 8 * 8 * (size_t)a.ncot));
+        if (wide)
+            hipLaunchKernelGGL((k_conv3<2, EPI, T>), grid, dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL((k_conv3<1, EPI, T>), grid, dim3(256), 0, s, a);
+    }
 }
 
 // y = relu(conv3x3(x) + bias); pool (may be null): also its 2 x 2 average
@@ -1300,6 +1307,10 @@ int mbrec_conv3x3_bf16(const uint16_t *x, const uint16_t *w, const float *bias, 
 {
     if (!x || !w || !y || N <= 0 || H <= 0 || W <= 0 || Cin % 32 || Cout % 32 || Cin <= 0 || Cout <= 0)
         return set_error(MBREC_ERR_ARG, "mbrec:args", "conv3x3_bf16: Cin and Cout must be positive multiples of 32");
+    // pixel and virtual column indices (at most two columns a pixel, one tile past the end) are 32-bit
+    constexpr size_t lim = ((size_t)1 << 30) - 64;
+    if ((size_t)N * H >= lim || (size_t)N * H * W >= lim)
+        return set_error(MBREC_ERR_ARG, "mbrec:args", "conv3x3_bf16: N * H * W must be below 2^30 - 64");
     // the kernel reads and writes 16- and 8-byte pieces: arrays at other addresses go through aligned copies
     hipStream_t s = (hipStream_t)stream;
     if (!relu && bias) return set_error(MBREC_ERR_ARG, "mbrec:args", "conv3x3_bf16: bias requires relu=1");
@@ -1320,8 +1331,9 @@ int mbrec_conv3x3_bf16(const uint16_t *x, const uint16_t *w, const float *bias, 
     a.y = fy.p;
     a.ys = Cout;
     a.bias = bias;
-    if (relu) conv_launch<kRelu>(a, s);
-    else conv_launch<kGrad>(a, s);   // plain convolution
+    const bool far = nx / 16 >= (size_t)INT32_MAX;   // slots beyond 32-bit indices
+    if (relu) far ? conv_launch<kRelu, long long>(a, s) : conv_launch<kRelu>(a, s);
+    else far ? conv_launch<kGrad, long long>(a, s) : conv_launch<kGrad>(a, s);   // plain convolution
     if (cy) MBREC_HIP(hipMemcpyAsync(y, cy, ny, hipMemcpyDeviceToDevice, s));
     for (void *q : {cx, cw, cy})
         if (q) MBREC_HIP(hipFreeAsync(q, s));

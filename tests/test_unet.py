@@ -292,3 +292,49 @@ def test_unet_ragged_grids_match_oracle(require_gpu, c, N, H, W):
         # to 2-3 % at these sizes (any order of the FP32 sums); a wrong tap, tile edge or
         # channel by far more
         assert rel_l2(grad[wo:bo + co], gw[wo:bo + co]) < 8e-2, name
+
+
+def test_conv3x3_bf16_size_check():
+    """Sizes beyond the kernel's 32-bit pixel indices are an error, found before any device call
+    (products that leave 64 bits among them); the pointers are never read."""
+    from mbrec import _lib
+    L = _lib.lib()
+    for N, H, W in [(1, 1 << 15, 1 << 15), (1 << 30, 1, 1), (1, 1, (1 << 31) - 1), (1 << 22, 1 << 22, 1 << 22)]:
+        assert L.mbrec_conv3x3_bf16(256, 256, None, 256, N, H, W, 32, 32, 1, None) == -1
+        assert b"2^30" in L.mbrec_last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Cout,relu", [(32, 1), (64, 0)])
+def test_conv3x3_bf16_beyond_32_bit_slots(require_gpu, Cout, relu):
+    """17 images of 2048^2 x 256 channels (36 GB): the last image starts at 16-byte slot 2^31, where a
+    32-bit index turns negative.  Its corners and the last rows before it against FP64, the images before
+    (zeros) exactly."""
+    import torch
+    from mbrec import _lib
+    print(f"conv3x3 far slots Cout={Cout}", flush=True)
+    N, H, W, Cin = 17, 2048, 2048, 256
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 64 GB of device memory")
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.zeros((N, H, W, Cin), dtype=torch.bfloat16, device="cuda")
+    x[N - 1].normal_(generator=g)
+    x[N - 2, H - 3:].normal_(generator=g)
+    w = _bf16_tensor(rng(8).standard_normal((Cout, 3, 3, Cin)) / np.sqrt(9 * Cin)).cuda()
+    y = torch.full((N, H, W, Cout), 7.0, dtype=torch.bfloat16, device="cuda")
+    _lib.check(_lib.lib().mbrec_conv3x3_bf16(x.data_ptr(), w.data_ptr(), None, y.data_ptr(), N, H, W, Cin, Cout, relu,
+                                             _lib.stream_handle()))
+    for n in (0, 7, N - 2):
+        assert (y[n, :H - 4] == 0).all()
+    k = 24
+    for n, hs, ws in [(N - 1, 0, 0), (N - 1, 0, W - k), (N - 1, H - k, 0), (N - 1, H - k, W - k), (N - 2, H - k, W - k)]:
+        pad = torch.zeros((k + 2, k + 2, Cin), dtype=torch.float64)     # the crop with its neighbours, zero outside
+        h0, h1, w0, w1 = max(hs - 1, 0), min(hs + k + 1, H), max(ws - 1, 0), min(ws + k + 1, W)
+        pad[h0 - hs + 1:h1 - hs + 1, w0 - ws + 1:w1 - ws + 1] = x[n, h0:h1, w0:w1].cpu().double()
+        want = torch.nn.functional.conv2d(pad.permute(2, 0, 1)[None], w.cpu().double().permute(0, 3, 1, 2))[0]
+        want = (torch.relu(want) if relu else want).permute(1, 2, 0).numpy()
+        got = y[n, hs:hs + k, ws:ws + k].float().cpu().numpy()
+        # outputs rounded to bfloat16 (2^-9 relative), FP32 sums of 9 Cin products below that
+        assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 1e-5)
+    del x, y
+    torch.cuda.empty_cache()
