@@ -45,7 +45,6 @@ __global__ void k_tv_load(const float *__restrict__ z, double *__restrict__ u, d
 constexpr int kNmMaxFactors = 24;
 constexpr int kNmLdsPoints = 2048;   // complex points per LDS buffer (two buffers: 64 KB)
 constexpr int kNmMaxN = kNmLdsPoints;
-constexpr int kNmIpPoints = 4096;    // complex points of an in-place transform (one buffer)
 
 struct NmFactors {
     int n;
@@ -118,8 +117,8 @@ __device__ double2 *nm_fft(double2 *a, double2 *b, int N, int C, const NmFactors
 // The same transform in place for N a product of 2, 3, 4, 5, 7 and 8: a thread takes whole
 // butterflies (p points read once, twiddled, transformed in registers), all reads of a stage before
 // its writes.  Against a thread per output (p reads and p twiddles each, two LDS buffers) the
-// passes of a 600^2 x 32 solve take 0.27 instead of 0.51 ms.  At most 4096 points for 512 threads (2048 for
-// 256), so KB butterflies per thread cover a stage.
+// passes of a 600^2 x 32 solve took 0.27 instead of 0.51 ms (six row pairs per workgroup).  At most
+// 4096 points for 512 threads (2048 for 256), so KB butterflies per thread cover a stage.
 __device__ __forceinline__ double2 nm_mul(double2 x, double2 w) { return make_double2(x.x * w.x - x.y * w.y, x.x * w.y + x.y * w.x); }
 __device__ __forceinline__ double2 nm_add(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ double2 nm_sub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
@@ -775,12 +774,17 @@ static int prox_setup(TvProx &T, hipStream_t s)   // after the scratch is there
     MBREC_HIP(hipMemcpyAsync(T.lam, lam.data(), sizeof(double) * N, hipMemcpyHostToDevice, s));
     MBREC_HIP(hipStreamSynchronize(s));
     T.nm.N = N;
-    // row pairs per workgroup: in place up to eight, as many as 4096 complex points hold (64 KB of LDS,
-    // two workgroups of 512 per CU; at 600^2 six, 96-byte runs in pass 2); else about 512 points
-    // between two buffers
+    // row pairs per workgroup: in place up to four within 2048 complex points (two above 682, within 4096:
+    // 64 KB of LDS, 512 threads), so that pass 2 moves runs of 32 to 64 bytes, but only as many as
+    // leave about 600 workgroups for the 256 CUs.  Whole call, 1 / 2 / 4 / 8 pairs (600^2: 1 / 2 / 3 / 6):
+    // 150^2 x 1 0.75 / 0.79 / 0.87 / 1.05 ms, x 32 1.63 / 1.36 / 1.22 / 1.33; 400^2 x 4 1.53 / 1.51 / 1.73 /
+    // 1.81, x 32 5.34 / 4.45 / 4.22 / 4.51; 600^2 x 4 2.57 / 2.37 / 2.55 / 2.57, x 32 10.9 / 9.1 / 9.0 / 9.3.
+    // Between two buffers: about 512 points
     T.ip = nm_factors_ip(N, T.nm.f);
+    const int pairs = (N + 1) / 2;
     if (T.ip)
-        T.nm.C = std::max(1, std::min({8, kNmIpPoints / N, (N + 1) / 2}));
+        T.nm.C = std::max(1, (int)std::min({(size_t)std::min(4, std::max(2, 2048 / N)), (size_t)pairs,
+                                            (size_t)pairs * T.B / 600}));
     else
         T.nm.C = std::max(1, std::min(4, 512 / N));
     if (!T.ip && !nm_factors(N, T.nm.f))

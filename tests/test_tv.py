@@ -238,3 +238,20 @@ def test_sb_itv2_transform_sizes(require_gpu, N):
         its.append(k)
         assert rel_l2(u[b].ravel(), ref) < 1e-6, b
     assert it == max(its)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,B", [(16, 90), (16, 400), (35, 80), (42, 90), (42, 120), (210, 12), (512, 16), (720, 4)])
+def test_sb_itv2_row_pairs_per_workgroup(require_gpu, N, B):
+    """Batches that give a workgroup of the in-place transform 1 to 4 row pairs, with and without a
+    remainder (8, 18, 21, 105, 256 and 360 pairs): three images in turn against the oracle."""
+    from mbrec.solvers import SB_ITV2
+    print(f"sb_itv2 row pairs N={N} B={B}", flush=True)
+    mus = np.array([0.2, 0.02, 1.5])
+    g = (rng(N).standard_normal((3, N, N)) + 2.0 * (np.arange(N) > N / 3)).astype(np.float32)
+    D = O.diff_oper(N)
+    ref = [O.sb_itv2(a.astype(np.float64).ravel(), m, D, exact=True) for a, m in zip(g, mus)]
+    u, it = SB_ITV2(np.resize(g, (B, N, N)), np.resize(mus, B))
+    assert it == max(k for _, k in ref)
+    for b in range(B):
+        assert rel_l2(u[b].ravel(), ref[b % 3][0]) < 1e-6, b
