@@ -109,6 +109,9 @@ int mbrec_plan_set_prefilter(mbrec_plan plan, const double *kz, int Kz, const do
 /* model_normalization_factor (MSOTmodel.m:271-287). */
 int mbrec_plan_set_sigma(mbrec_plan plan, double sigma);
 int mbrec_plan_destroy(mbrec_plan plan);
+/* Gives back the scratch memory that the total-variation entry points keep between calls (at most
+ * 1 GB per device, all devices), as mbrec_plan_destroy does too. */
+void mbrec_release_scratch(void);
 /* Bytes the plan holds on the device (tables + workspace). */
 size_t mbrec_plan_device_bytes(mbrec_plan plan);
 /* Fixed-point travel-time format: number of fractional bits. */

@@ -37,7 +37,7 @@ static int dalloc(T **ptr, size_t n, size_t *acc)
 {
     *ptr = nullptr;
     if (n == 0) n = 1;
-    hipError_t e = hipMalloc((void **)ptr, n * sizeof(T));
+    hipError_t e = device_malloc((void **)ptr, n * sizeof(T));
     if (e != hipSuccess) {
         (void)hipGetLastError();
         return set_error(MBREC_ERR_HIP, "mbrec:alloc", "hipMalloc of %zu bytes failed: %s",
@@ -97,10 +97,18 @@ hipError_t scratch_malloc(void **p, size_t bytes, hipStream_t s)
 
 void scratch_trim()
 {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kPoolDevices) return;
     std::lock_guard<std::mutex> lk(g_pool_mu);
-    if (g_pool[dev] && hipMemPoolTrimTo(g_pool[dev], 0) != hipSuccess) (void)hipGetLastError();
+    for (hipMemPool_t pool : g_pool)
+        if (pool && hipMemPoolTrimTo(pool, 0) != hipSuccess) (void)hipGetLastError();
+}
+
+hipError_t device_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    scratch_trim();
+    return hipMalloc(p, bytes);
 }
 
 int ensure_work(Plan *p, int B)
@@ -1151,6 +1159,8 @@ int mbrec_plan_set_sigma(mbrec_plan h, double sigma)
     h->p.sigma = sigma;
     return MBREC_OK;
 }
+
+void mbrec_release_scratch(void) { scratch_trim(); }
 
 int mbrec_plan_destroy(mbrec_plan h)
 {

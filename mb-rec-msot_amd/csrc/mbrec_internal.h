@@ -181,13 +181,16 @@ struct Plan {
 
 // Stream-ordered scratch (freed with hipFreeAsync) from a pool of the library's own, one per device,
 // which keeps up to 1 GB of released memory between calls, so that a call's allocations do not map
-// fresh memory each time; scratch_trim gives it back (mbrec_plan_destroy does).  The pool's own
+// fresh memory each time.  scratch_trim gives every device's back: mbrec_plan_destroy,
+// mbrec_release_scratch and an allocation of the library's that finds no memory call it.  The pool's own
 // ordering makes the memory safe to share between streams and threads.  1 GB holds the TV prox of
 // 32 images of 600^2 (0.65 GB), whose hipMalloc / hipFree took 1.5 ms a call.
 constexpr int kPoolDevices = 64;
 constexpr unsigned long long kPoolKeep = 1ull << 30;
 hipError_t scratch_malloc(void **p, size_t bytes, hipStream_t s);
 void scratch_trim();
+// hipMalloc, once more without the kept scratch where the device has no memory left
+hipError_t device_malloc(void **p, size_t bytes);
 
 static inline int batch_stride(int B) { return B <= 1 ? 1 : (B + 3) / 4 * 4; }
 

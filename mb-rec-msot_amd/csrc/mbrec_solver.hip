@@ -395,7 +395,7 @@ struct Workspace {
     template <typename T>
     int alloc(T **p, size_t n)
     {
-        hipError_t e = hipMalloc((void **)p, (n ? n : 1) * sizeof(T));
+        hipError_t e = device_malloc((void **)p, (n ? n : 1) * sizeof(T));
         if (e != hipSuccess) {
             (void)hipGetLastError();
             return set_error(MBREC_ERR_HIP, "mbrec:alloc", "solver workspace allocation failed: %s",

@@ -785,7 +785,7 @@ static void free_ws(UNet *u)
 
 static int walloc(UNet *u, void **p, size_t bytes)
 {
-    if (hipMalloc(p, std::max<size_t>(bytes, 16)) != hipSuccess) {
+    if (device_malloc(p, std::max<size_t>(bytes, 16)) != hipSuccess) {
         (void)hipGetLastError();
         return set_error(MBREC_ERR_HIP, "mbrec:oom", "unet: device allocation of %zu bytes failed", bytes);
     }

@@ -10,7 +10,12 @@ from .probe import Probe  # noqa: F401
 
 __all__ = ["MbrecError", "lib", "LIB_PATH", "Discretization", "Probe", "MSOTmodel",
            "define_model_for_reconstruction", "rec_nn_with_L2_reg", "rec_nn_with_L1_eye_reg", "rec_nn_with_TV_reg", "forwardMex", "transposeMex",
-           "forwardDelayAndSumMex", "transposeDelayAndSumMex"]
+           "forwardDelayAndSumMex", "transposeDelayAndSumMex", "release_scratch"]
+
+
+def release_scratch():
+    """Gives back the device memory that the total-variation solvers keep between calls (at most 1 GB)."""
+    lib().mbrec_release_scratch()
 
 
 def __getattr__(name):

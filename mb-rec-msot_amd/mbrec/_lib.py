@@ -44,6 +44,7 @@ SIGNATURES = [
     ("mbrec_plan_set_prefilter", C.c_int, [c_void_p, c_void_p, C.c_int, c_void_p, C.c_int]),
     ("mbrec_plan_set_sigma", C.c_int, [c_void_p, C.c_double]),
     ("mbrec_plan_destroy", C.c_int, [c_void_p]),
+    ("mbrec_release_scratch", None, []),
     ("mbrec_plan_device_bytes", C.c_size_t, [c_void_p]),
     ("mbrec_plan_tau_frac_bits", C.c_int, [c_void_p]),
     ("mbrec_plan_autotune", C.c_int, [c_void_p, C.c_int, C.c_int, c_void_p, c_int32_p]),

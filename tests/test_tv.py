@@ -255,3 +255,32 @@ def test_sb_itv2_row_pairs_per_workgroup(require_gpu, N, B):
     assert it == max(k for _, k in ref)
     for b in range(B):
         assert rel_l2(u[b].ravel(), ref[b % 3][0]) < 1e-6, b
+
+
+@pytest.mark.gpu
+def test_tv_scratch_is_given_back(require_gpu):
+    """SB_ITV2 keeps its scratch between calls, within 1 GB; release_scratch and the end of any plan
+    give it back."""
+    import gc
+    import torch
+    import mbrec
+    from mbrec.model import DevicePlan
+    from mbrec.solvers import SB_ITV2
+    g = torch.rand((16, 400, 400), device="cuda")         # 20 MB of each of seven FP64 arrays
+    mu = np.full(16, 0.05)
+    SB_ITV2(g, mu)
+    tt = np.full((3, 20), 10.0)
+    for release in ("call", "plan"):
+        gc.collect()
+        torch.cuda.synchronize()
+        mbrec.release_scratch()
+        torch.cuda.empty_cache()
+        free = torch.cuda.mem_get_info()[0]
+        plan = DevicePlan(5, 4, 3, 40, 2.0, tt)
+        SB_ITV2(g, mu)
+        torch.cuda.empty_cache()
+        kept = free - torch.cuda.mem_get_info()[0]
+        assert 7 * 16 * 160000 * 8 <= kept <= (1 << 30) + (64 << 20)
+        mbrec.release_scratch() if release == "call" else plan.close()
+        plan.close()
+        assert free - torch.cuda.mem_get_info()[0] < 32 << 20
