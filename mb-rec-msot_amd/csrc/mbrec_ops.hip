@@ -1430,7 +1430,8 @@ __global__ __launch_bounds__(256) void k_fwd_pull_bl(const int2 *__restrict__ re
 // one detector, so bin offsets and records are uniform over the wave and live
 // in scalar registers.  Per bin, its records are consumed in runs of U whose
 // image rows are all loaded before any is accumulated (records past the bin's
-// end read the zero padding after the table with weight 0).
+// end, the next bin's or the zero padding after the table, count as a pixel of value 0,
+// whatever theirs is: a weight of 0 would let an infinite one into this bin).
 template <int U>
 __global__ __launch_bounds__(256) void k_fwd_pull_wu(const int2 *__restrict__ rec, const int32_t *__restrict__ off,
                                                      const float *__restrict__ imgI, float *__restrict__ bins, int NB,
@@ -1473,10 +1474,9 @@ __global__ __launch_bounds__(256) void k_fwd_pull_wu(const int2 *__restrict__ re
             for (int u = 0; u < U; ++u) cv[u] = cb[(size_t)e[u].x * Bp];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const bool in = r + u < r1;
-                const float uu = in ? __int_as_float(e[u].y) : 0.0f;
-                s0 = fmaf(in ? 1.0f - uu : 0.0f, cv[u], s0);
-                s1 = fmaf(uu, cv[u], s1);
+                const float uu = __int_as_float(e[u].y), c = r + u < r1 ? cv[u] : 0.0f;
+                s0 = fmaf(1.0f - uu, c, s0);
+                s1 = fmaf(uu, c, s1);
             }
         }
         if (b < Bp) dst[(size_t)j * Bp] = s0 + prev;
@@ -1488,7 +1488,7 @@ __global__ __launch_bounds__(256) void k_fwd_pull_wu(const int2 *__restrict__ re
 // Wave-uniform pull with raw-buffer image-row loads: records are read with
 // scalar loads, each image row at a scalar byte offset (no per-pair address
 // arithmetic in vector registers); full runs of U records carry no tests and
-// the tail of a bin runs once more with weights zeroed past its end.  The image
+// the tail of a bin runs once more with the values past its end taken as 0.  The image
 // is read as a raw buffer with 32-bit offsets: P * Bp floats below 2^31 bytes
 // (checked by the launcher).
 template <int U>
@@ -1544,7 +1544,7 @@ __global__ __launch_bounds__(256) void k_fwd_pull_wt(const int2 *__restrict__ re
                 s1 = fmaf(uu, cv[u], s1);
             }
         }
-        if (r < r1) {   // tail: records past r1 (next bin's, or the zero pad) get weight 0
+        if (r < r1) {   // tail: the values of records past r1 (next bin's, or the zero pad) count as 0
             int2 e[U];
             float cv[U];
 #pragma unroll
@@ -1553,10 +1553,9 @@ __global__ __launch_bounds__(256) void k_fwd_pull_wt(const int2 *__restrict__ re
             for (int u = 0; u < U; ++u) cv[u] = ld(e[u].x);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const bool in = r + u < r1;
-                const float uu = in ? __int_as_float(e[u].y) : 0.0f;
-                s0 = fmaf(in ? 1.0f - uu : 0.0f, cv[u], s0);
-                s1 = fmaf(uu, cv[u], s1);
+                const float uu = __int_as_float(e[u].y), c = r + u < r1 ? cv[u] : 0.0f;
+                s0 = fmaf(1.0f - uu, c, s0);
+                s1 = fmaf(uu, c, s1);
             }
         }
         if (b < Bp) dst[(size_t)j * Bp] = s0 + prev;

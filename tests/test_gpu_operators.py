@@ -337,6 +337,36 @@ def test_default_batch_forms_match_oracle(B, smooth):
     assert rel_l2(xt.reshape(B, -1), xto) < TOL_OP
 
 
+@pytest.mark.parametrize("B", [12, 13, 28, 33, 64, 70])
+def test_forward_keeps_non_finite_pixels_apart(B):
+    """Infinite and NaN pixels reach the samples of their own pairs only, and their own sinogram only:
+    every batch form against the form with a thread per bin (forward choice 1), which reads the
+    records of its bin and no others."""
+    import torch
+    _log(f"non-finite pixels B={B}")
+    Nz, Nx, D, nT = 13, 11, 24, 150
+    plan, tt, _, _ = _plan_problem(Nz, Nx, D, nT, 2.6666666666666665, seed=90)
+    x = rng(91).uniform(0, 1, (B, Nx, Nz)).astype(np.float32)
+    for k, (b, v) in enumerate([(0, np.inf), (1, -np.inf), (5, np.nan), (B - 1, np.inf), (B - 1, np.nan)]):
+        x[b, 3 + k, 4] = v
+    xd = torch.tensor(x).cuda()
+    plan.set_launch(B, -1, 1)
+    want = plan.forward(xd, model=False).cpu().numpy()
+    bad = ~np.isfinite(want)
+    assert bad[[0, 1, 5, B - 1]].any(axis=(1, 2)).all() and not bad[[2, 3, 4]].any() and bad.mean() < 0.05
+    ran = 0
+    for c in [0] + [-lb - 100 * mode for mode in range(12) for lb in (16, 32, 64)]:
+        try:
+            plan.set_launch(B, -1, c)
+        except Exception:
+            continue
+        ran += c < 0
+        y = plan.forward(xd, model=False).cpu().numpy()
+        assert np.array_equal(~np.isfinite(y), bad), c
+        assert rel_l2(y[~bad], want[~bad]) < TOL_OP, c
+    assert B == 12 or ran >= 10
+
+
 def test_one_sinogram_tile_variants_match_oracle():
     """Every one-sinogram tile form on a real arc geometry (the tile windows fit the LDS only
     for smooth travel times): forward choices 2, 3 (record streaming), 5, 6, 7 (tile form, thread
