@@ -146,7 +146,7 @@ int mbrec_plan_autotune(mbrec_plan plan, int B, int reps, mbrec_stream s, int *c
  * -(LB + 100 mode) batch-lane with lane groups LB and mode 0 (plain order), 1
  * (XCD-aware order), 2 (XCD-aware, 16 pairs in flight); -364 / -464 / -564 /
  * -664 / -764 / -864 wave-uniform, -964 / -1064 / -1164 wave-uniform with raw
- * buffer loads (bins per wave and rows in flight differ).  Invalid choices are
+ * buffer loads (bins per wave and rows in flight differ; batches of 9 and more).  Invalid choices are
  * rejected (mbrec:args). */
 int mbrec_plan_set_launch(mbrec_plan plan, int B, int gather_variant, int scatter_choice);
 /* Kernel of the IR convolution / correlation stage (MSOTmodel.m:259-269, FFTs in FP64

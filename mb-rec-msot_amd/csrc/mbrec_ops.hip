@@ -3326,9 +3326,9 @@ static bool pull_choice_ok(const Plan *p, int c, int Bp)
         int cap = 16;
         while (cap < Bp) cap *= 2;
         if (mode >= 9)   // raw-buffer image rows: 32-bit byte offsets
-            return Bp >= 16 && lb == 64 && mode <= 11 && sizeof(float) * (size_t)p->P * Bp < ((size_t)1 << 31);
-        if (mode >= 3)   // wave-uniform runs: lane groups of 64 only
-            return Bp >= 16 && lb == 64 && mode <= 8;
+            return Bp >= 12 && lb == 64 && mode <= 11 && sizeof(float) * (size_t)p->P * Bp < ((size_t)1 << 31);
+        if (mode >= 3)   // wave-uniform runs: lane groups of 64 only (the default from 12 sinograms on)
+            return Bp >= 12 && lb == 64 && mode <= 8;
         return Bp >= 16 && (lb == 16 || lb == 32 || lb == 64) && lb <= cap && mode <= 2;
     }
     return false;
