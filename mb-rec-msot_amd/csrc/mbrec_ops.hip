@@ -2619,14 +2619,18 @@ __global__ __launch_bounds__(1024, LB <= 32 ? 8 : 4) void k_gather_ta(
                 rt, (__attribute__((address_space(3))) void *)(bb + L::RS * LB + 256 * wv), 16, 16 * lane,
                 (int)((((size_t)tile * D + d) * 256 + 128 * wv) * sizeof(int2)), 0, 0);
     };
-    // sums of eight detectors in FP32, added up in FP64 with LB <= 32 (as close to the exact sum as the
-    // compensated sums of the record- and batch-lane forms: 3.1e-7 against 3.0e-7 of the operator at
-    // 301 x 333 x 28).  64 registers at most there: 66 would leave one workgroup per CU (0.41 / 0.29 ms)
-    using Sum = std::conditional_t<(LB <= 32), double, float>;
-    Sum acc[NP];
-    float part[NP];
+    // the sum over the detectors: in FP64 with LB <= 32, its partial images too, so that the only
+    // rounding is the last one, as with the compensated sums of the record- and batch-lane forms (FP32 sums
+    // of eight detectors and FP32 partial images: 1.4 to 1.6 times their error, and 4 % faster).  64
+    // registers at most there (58 used, none spilled): 66 would leave one workgroup per CU (0.41 / 0.29 ms
+    // at 301 x 333 x 28).  Else FP32 sums of eight detectors
+    constexpr bool F64 = LB <= 32;
+    std::conditional_t<F64, double, float> acc[NP];
+    float part[F64 ? 1 : NP];
 #pragma unroll
-    for (int k = 0; k < NP; ++k) acc[k] = part[k] = 0.0f;
+    for (int k = 0; k < NP; ++k) acc[k] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < (F64 ? 1 : NP); ++k) part[k] = 0.0f;
     // one detector: wait for its loads, barrier, start the fill two ahead, interpolate
     auto step = [&](int d, const float *rd, float *wr) __attribute__((always_inline)) {
         if (d + 1 < dend) {   // this wave's loads for d are done (those for d + 1 may be in flight)
@@ -2658,13 +2662,18 @@ __global__ __launch_bounds__(1024, LB <= 32 ? 8 : 4) void k_gather_ta(
             g1[2 * k2 + 1] = wb[e.z * LB + LB];
             uu[2 * k2 + 1] = __int_as_float(e.w);
         }
+        if constexpr (F64) {
 #pragma unroll
-        for (int k = 0; k < NP; ++k) part[k] += fmaf(uu[k], g1[k] - g0[k], g0[k]);
-        if (((d - dbeg) & 7) == 7) {
+            for (int k = 0; k < NP; ++k) acc[k] += (double)fmaf(uu[k], g1[k] - g0[k], g0[k]);
+        } else {
 #pragma unroll
-            for (int k = 0; k < NP; ++k) {
-                acc[k] += part[k];
-                part[k] = 0.0f;
+            for (int k = 0; k < NP; ++k) part[k] += fmaf(uu[k], g1[k] - g0[k], g0[k]);
+            if (((d - dbeg) & 7) == 7) {
+#pragma unroll
+                for (int k = 0; k < NP; ++k) {
+                    acc[k] += part[k];
+                    part[k] = 0.0f;
+                }
             }
         }
     };
@@ -2687,13 +2696,13 @@ __global__ __launch_bounds__(1024, LB <= 32 ? 8 : 4) void k_gather_ta(
     if (b >= B) return;
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-        const float v = (float)(acc[k] + part[k]);
+        const auto v = F64 ? acc[k] : acc[k] + part[F64 ? 0 : k];
         const int px = pix[(size_t)tile * 256 + 16 * wv + (lane / LB) * NP + k];
         if (px < 0) continue;
         if (G > 1)
-            out[((size_t)grp * B + b) * P + px] = v;
+            reinterpret_cast<std::conditional_t<F64, double, float> *>(out)[((size_t)grp * B + b) * P + px] = v;
         else
-            out[(size_t)b * P + px] = scale * v;
+            out[(size_t)b * P + px] = scale * (float)v;
     }
 }
 
@@ -3219,16 +3228,16 @@ __global__ __launch_bounds__(256) void k_gather_tas1(const int4 *__restrict__ st
         out[px] = scale * (acc + part);
 }
 
-// out[b][x] = scale * sum of the NP partial images (fixed order)
-template <int NP>
-__global__ __launch_bounds__(256) void k_sum_parts(const float *__restrict__ part, float *__restrict__ out,
+// out[b][x] = scale * sum of the NP partial images (fixed order; FP64 images are rounded once, after it)
+template <int NP, typename T = float>
+__global__ __launch_bounds__(256) void k_sum_parts(const T *__restrict__ part, float *__restrict__ out,
                                                    size_t n, float scale)
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        float s = 0.0f;
+        T s = 0;
 #pragma unroll
         for (int k = 0; k < NP; ++k) s += part[(size_t)k * n + i];
-        out[i] = scale * s;
+        out[i] = scale * (float)s;
     }
 }
 
@@ -4218,9 +4227,11 @@ static void gather_ta_n(Plan *p, float *img, int B, int Bp, float scale, hipStre
                        p->d_bins, G > 1 ? p->d_gpart : img, p->D, p->geom.NB, p->P, B, Bp, scale, bytes, tbytes,
                        (const int32_t *)p->d_tord);
     if (G > 1) {
+        using Part = std::conditional_t<(LB <= 32), double, float>;
+        static_assert(G * sizeof(Part) <= 8 * sizeof(float), "partial images fit d_gpart");
         const size_t n = (size_t)B * p->P;
-        hipLaunchKernelGGL(k_sum_parts<G>, dim3(std::min<size_t>(4096, (n + 255) / 256)), dim3(256), 0, s,
-                           (const float *)p->d_gpart, img, n, scale);
+        hipLaunchKernelGGL((k_sum_parts<G, Part>), dim3(std::min<size_t>(4096, (n + 255) / 256)), dim3(256), 0, s,
+                           (const Part *)p->d_gpart, img, n, scale);
     }
 }
 
@@ -4445,9 +4456,9 @@ static int default_gather_variant(const Plan *p, int Bp)
     if (!p->use_sir && Bp >= 12 && Bp <= 64) {
         // LDS tile gather with 32 sinograms per workgroup (16 up to Bp = 16) and two or more workgroups
         // per CU, in two detector groups, four where those leave CUs without one.  Measured, stage time
-        // against the former choices: 301 x 333 x 28 0.29 / 1.22 ms (the 64-sinogram form 0.56), x 16
-        // 0.18 / 0.57 ms, x 12 0.18 / 0.43 ms (x 8: 0.17 / 0.13, so Bp = 8 stays), 400^2 x 64
-        // 0.74 / 0.84 ms (x 100: 2.4 / 1.7, so larger batches stay).
+        // against the former choices: 301 x 333 x 28 0.30 / 1.22 ms (the 64-sinogram form 0.60), x 13
+        // 0.19 / 0.57 ms, x 9 0.18 / 0.43 ms (x 8: 0.17 / 0.13, so Bp = 8 stays), 400^2 x 64
+        // 0.78 / 0.84 ms (x 100: 2.4 / 1.7, so larger batches stay).
         const bool small = Bp <= 16;
         const int tiles = p->Pd / 256, chunks = small ? 1 : (Bp + 31) / 32;
         const bool few = tiles * chunks * 2 < (small ? 1024 : 512);

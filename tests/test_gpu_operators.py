@@ -378,6 +378,26 @@ def test_forward_keeps_non_finite_pixels_apart(B):
     assert ran >= 9
 
 
+@pytest.mark.parametrize("B", [13, 28, 64])
+def test_batch_gather_sums_as_close_as_compensated(B):
+    """The LDS gathers of batches without SIR (55 to 58) add up 256 detectors of one sign: their distance to
+    the FP64 oracle is no larger than that of the compensated forms (2: record lanes, 7: batch lanes);
+    what those share, the 32-bit interpolation weights, allows 1 % between them."""
+    import torch
+    _log(f"gather sums B={B}")
+    m = _geometry_model(57, 70, 256, 700, 1e-4, sir=False, sigma=1.0)
+    tt, R = _oracle_of(m).tt.T, _oracle_of(m).R
+    sg = 0.5 + rng(36).uniform(0, 1, (B, 256, 700))
+    ref = O.transpose_das(np.transpose(sg, (0, 2, 1)), tt, R)
+    sd = torch.tensor(sg, dtype=torch.float32).cuda()
+    err = {}
+    for v in (2, 7, 55, 56, 57, 58):
+        m.plan.set_launch(B, v, 0)
+        err[v] = rel_l2(m.plan.transpose(sd, model=False).cpu().numpy().reshape(B, -1), ref)
+    print(B, {k: f"{e:.3e}" for k, e in err.items()}, flush=True)
+    assert max(err[v] for v in (55, 56, 57, 58)) <= 1.01 * min(err[2], err[7])
+
+
 def test_one_sinogram_tile_variants_match_oracle():
     """Every one-sinogram tile form on a real arc geometry (the tile windows fit the LDS only
     for smooth travel times): forward choices 2, 3 (record streaming), 5, 6, 7 (tile form, thread
