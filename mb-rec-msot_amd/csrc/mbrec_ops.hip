@@ -2839,30 +2839,37 @@ __global__ __launch_bounds__(1024) void k_gather_tas(const int4 *__restrict__ st
 // SIR transpose for batches on the FP32 matrix cores: WG = 8 waves, one 256-slot tile x
 // LB = 16 NCB sinograms x one of G detector groups.  The tile's pairs with a detector come in
 // groups of at most 16 that share a phase and a window of 32 samples (build_sir_groups), so a
-// group is a product [16 pairs x 32 samples] x [32 samples x LB] of weights and bins, once with
-// weights w (1 - u) and the phase's bin rows and once with w u and the next rows, summed in
-// one accumulator: 16 NCB products 16x16x4.  The sample order is free: lane group q holds samples
+// group is a product [16 pairs x 32 samples] x [32 samples x LB] of weights and bins, once with the
+// phase's bin rows and once with the next rows: 16 NCB products 16x16x4; a pair's sum is the first plus u
+// times their difference (u put into the weights beforehand cost a rounding per tap).
+// The sample order is free: lane group q holds samples
 // 8 q + 0..7, so a pair's weights are two 16-byte loads per lane (4-byte aligned); odd lane
 // groups take them in swapped pairs, which puts their bin rows on the other 32 LDS banks.
 // Per detector the tile's bin rows are copied memory -> LDS once; the results go to the pixels'
-// sums in LDS (every pixel once per detector), which move to registers every eight detectors.
+// sums in LDS (every pixel once per detector): FP64 with NCB = 1, and FP64 partial images, where
+// the compensated record-lane form ran before (300^2 x 8: 2.4e-7 from 64 bits, 2.6e-7 there, 2.9e-7 with
+// FP32 sums); with NCB = 2 FP32, moved to FP32 registers every eight detectors, as k_gather_tas.
 // Two workgroups share a CU, one waiting for its rows and weights while the other multiplies.
 // Bound by the matrix cores: about 18 groups of 1024 cycles (NCB = 2) per tile and detector, at
-// 400^2 x 64 2.4 of 4.3 ms; the rest is the two barriers per detector.  Gather stage against the
+// 400^2 x 64 2.4 of 4.4 ms; the rest is the two barriers per detector.  Gather stage against the
 // vector form k_gather_tas (two FMAs and two lane reads per tap; it remains for windows that do
-// not fit the groups): 400^2 x 64 7.7 -> 4.3 ms, 300^2 x 28 4.3 -> 1.33 ms, x 4 1.66 (record lanes)
-// -> 0.80 ms.  The XCD order cut L2 misses from 26 to 8 GB at 400^2 x 64 (4.7 -> 4.5 ms).
+// not fit the groups): 400^2 x 64 7.7 -> 4.4 ms, 300^2 x 28 4.6 -> 1.5 ms, x 4 1.88 (record lanes)
+// -> 0.93 ms.  The XCD order cut L2 misses from 26 to 8 GB at 400^2 x 64 (4.7 -> 4.5 ms).
+template <int G, int NCB>
+using SgPart = std::conditional_t<(G <= 4 && NCB == 1), double, float>;   // partial images, at most 32 bytes a pixel
+
 template <int G, int NCH, int NCB>
 __global__ __launch_bounds__(512, 4) void k_gather_sg(const int32_t *__restrict__ hdr, const int2 *__restrict__ ent,
                                                       const uint32_t *__restrict__ slots,
                                                       const int32_t *__restrict__ pix, const float *__restrict__ bins,
-                                                      const float *__restrict__ sirw, float *__restrict__ out,
+                                                      const float *__restrict__ sirw, SgPart<G, NCB> *__restrict__ out,
                                                       const int32_t *__restrict__ tord, int ntile, int tlen, int nbc,
-                                                      int D, int NB, int P, int B, int Bp, float scale)
+                                                      int D, int NB, int P, int B, int Bp)
 {
     constexpr int LB = 16 * NCB, ROWS = 64 * NCH, RPL = 256 / LB, NV = 256 * LB / 512, GW = kSgGroups / 8;
+    using Sum = std::conditional_t<NCB == 1, double, float>;   // the pixels' sums in LDS
     __shared__ __attribute__((aligned(16))) float s_row[ROWS * LB];
-    __shared__ float s_acc[257 * LB];
+    __shared__ Sum s_acc[257 * LB];
     // blocks of an XCD (every eighth): the column chunks of a tile side by side, then the next tile of
     // the XCD's compact run, then the next detector group
     const int r_ = blockIdx.x >> 3, tj = (r_ / nbc) % tlen, b0 = (r_ % nbc) * LB, grp = r_ / nbc / tlen;
@@ -2873,11 +2880,11 @@ __global__ __launch_bounds__(512, 4) void k_gather_sg(const int32_t *__restrict_
     const int DG = (D + G - 1) / G, dbeg = grp * DG, dend = min(D, dbeg + DG);
     const int last_row = D * NB + 1;   // of the bins (two zero rows after the detectors')
     const int lrow = lane / (LB / 4), lcol = min(b0 + 4 * (lane % (LB / 4)), Bp - 4);   // staging: row of a load, columns
-    float tot[NV];
+    float tot[NCB == 1 ? 1 : NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-        tot[k] = 0.0f;
-        s_acc[tid + 512 * k] = 0.0f;
+        if (NCB > 1) tot[NCB == 1 ? 0 : k] = 0.0f;
+        s_acc[tid + 512 * k] = 0;
     }
     int2 e[GW];
     uint32_t sl[GW];
@@ -2924,13 +2931,12 @@ __global__ __launch_bounds__(512, 4) void k_gather_sg(const int32_t *__restrict_
             const int g = wv + 8 * k;
             if (g >= ng) break;   // uniform
             const int gh = h[2 + g], cnt = gh >> 16;
-            const float u0 = 1.0f - u[k], u1 = u[k];
             // LDS row of lane group q's sample 8 q (+ 1 for odd groups, whose sample order is swapped in pairs)
             const float *row = s_row + (3 * ((gh & 255) + 8 * q) + ((gh >> 8) & 255)) * LB + i;
             const float *re = row + odd * 3 * LB, *ro = row + (1 - odd) * 3 * LB;
-            f32x4 acc[NCB];
+            f32x4 acc[2][NCB];
 #pragma unroll
-            for (int c = 0; c < NCB; ++c) acc[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int c = 0; c < NCB; ++c) acc[0][c] = acc[1][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             // bin rows of four samples at a time, the next four in flight during their products (the barriers
             // keep the compiler from moving every read next to its product)
             float rv[2][4][2][NCB];
@@ -2950,53 +2956,55 @@ __global__ __launch_bounds__(512, 4) void k_gather_sg(const int32_t *__restrict_
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const float wa = w[k][hf][t], wb = w[k][hf][t ^ 1], ws = odd ? wb : wa;
-                    const float a0 = ws * u0, a1 = ws * u1;
 #pragma unroll
-                    for (int c = 0; c < NCB; ++c)
-                        acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, rv[hf][t][0][c], acc[c], 0, 0, 0);
+                    for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int c = 0; c < NCB; ++c)
-                        acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, rv[hf][t][1][c], acc[c], 0, 0, 0);
+                        for (int c = 0; c < NCB; ++c)
+                            acc[j][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(ws, rv[hf][t][j][c], acc[j][c], 0, 0, 0);
                 }
             };
             read(0);
             read(1);
             __builtin_amdgcn_sched_barrier(0);
             mul(0);
-            mul(1);
-            __builtin_amdgcn_sched_barrier(0);
             // lane: sinogram i (+ 16 c), pairs 4 q + r (past the group's end: to a row that nobody reads)
-            float *px[4], pv[4][NCB];
+            Sum *px[4], pv[4][NCB];
+            float ur[4], v[4][NCB];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 px[r] = s_acc + (4 * q + r < cnt ? (slc[k] >> 8 * r) & 255 : 256) * LB + i;
+                ur[r] = __shfl(u[k], 4 * q + r);
 #pragma unroll
                 for (int c = 0; c < NCB; ++c) pv[r][c] = px[r][16 * c];
             }
+            __builtin_amdgcn_sched_barrier(0);
+            mul(1);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
-                for (int c = 0; c < NCB; ++c) px[r][16 * c] = pv[r][c] + acc[c][r];
+                for (int c = 0; c < NCB; ++c) v[r][c] = fmaf(ur[r], acc[1][c][r] - acc[0][c][r], acc[0][c][r]);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int c = 0; c < NCB; ++c) px[r][16 * c] = pv[r][c] + v[r][c];
         }
-        if (((d - dbeg) & 7) == 7 || d + 1 == dend) {
+        if (NCB > 1 && (((d - dbeg) & 7) == 7 || d + 1 == dend)) {
             __syncthreads();
 #pragma unroll
             for (int k = 0; k < NV; ++k) {   // read and cleared by the same thread, before the barriers of the next detector
-                tot[k] += s_acc[tid + 512 * k];
-                s_acc[tid + 512 * k] = 0.0f;
+                tot[NCB == 1 ? 0 : k] += s_acc[tid + 512 * k];
+                s_acc[tid + 512 * k] = 0;
             }
         }
     }
+    if (NCB == 1) __syncthreads();
     const int b = b0 + tid % LB;
     if (b >= B) return;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         const int px = pix[(size_t)tile * 256 + tid / LB + (512 / LB) * k];
-        if (px < 0) continue;
-        if (G > 1)
-            out[((size_t)grp * B + b) * P + px] = tot[k];
-        else
-            out[(size_t)b * P + px] = scale * tot[k];
+        if (px >= 0) out[((size_t)grp * B + b) * P + px] = NCB == 1 ? s_acc[tid + 512 * k] : tot[NCB == 1 ? 0 : k];
     }
 }
 
@@ -4278,11 +4286,12 @@ static void gather_sg_n(Plan *p, float *img, int B, int Bp, float scale, hipStre
     const int nbc = (Bp + 16 * NCB - 1) / (16 * NCB), ntile = p->Pd / 256;
     const int tlen = p->d_tord ? p->tile_launch / 8 : (ntile + 7) / 8;   // tiles per XCD
     hipLaunchKernelGGL((k_gather_sg<G, NCH, NCB>), dim3(8 * tlen * G * nbc), dim3(512), 0, s, p->d_sghdr, p->d_sgent,
-                       p->d_sgslot, p->d_pix, p->d_bins, p->d_sirw, p->d_gpart, (const int32_t *)p->d_tord, ntile, tlen, nbc,
-                       p->D, p->geom.NB, p->P, B, Bp, scale);
+                       p->d_sgslot, p->d_pix, p->d_bins, p->d_sirw, (SgPart<G, NCB> *)p->d_gpart,
+                       (const int32_t *)p->d_tord, ntile, tlen, nbc, p->D, p->geom.NB, p->P, B, Bp);
+    static_assert(G * sizeof(SgPart<G, NCB>) <= 8 * sizeof(float), "partial images fit d_gpart");
     const size_t n = (size_t)B * p->P;
-    hipLaunchKernelGGL(k_sum_parts<G>, dim3(std::min<size_t>(4096, (n + 255) / 256)), dim3(256), 0, s,
-                       (const float *)p->d_gpart, img, n, scale);
+    hipLaunchKernelGGL((k_sum_parts<G, SgPart<G, NCB>>), dim3(std::min<size_t>(4096, (n + 255) / 256)), dim3(256), 0, s,
+                       (const SgPart<G, NCB> *)p->d_gpart, img, n, scale);
 }
 
 template <int G, int NCB>

@@ -398,6 +398,27 @@ def test_batch_gather_sums_as_close_as_compensated(B):
     assert max(err[v] for v in (55, 56, 57, 58)) <= 1.01 * min(err[2], err[7])
 
 
+@pytest.mark.parametrize("B,v", [(4, 61), (8, 61), (16, 61), (17, 59), (28, 59), (64, 59)])
+def test_sir_batch_gather_sums_as_close_as_before(B, v):
+    """The matrix-core SIR transpose adds up 75 detectors of one sign: its distance to the FP64 oracle is no
+    larger than that of the form it replaces for the batch, compensated record lanes (2) up to 16
+    sinograms, the vector tile form (39) above; 1 % for what those share."""
+    import torch
+    _log(f"SIR gather sums B={B}")
+    m = _geometry_model(37, 40, 75, 700, 1e-4, sir=True, sigma=1.0)
+    tt, d = _oracle_of(m).tt.T, m.Data
+    sg = 0.5 + rng(37).uniform(0, 1, (B, 75, 700))
+    ref = O.transpose_sir(np.transpose(sg, (0, 2, 1)), d.SPMRIndices.reshape(75, -1).T, tt, d.SPMR.T,
+                          d.SPMRTimestepIndexStartAndEnd.T, _oracle_of(m).R)
+    sd = torch.tensor(sg, dtype=torch.float32).cuda()
+    err = {}
+    for k in (-1, v, 2 if B <= 16 else 39):
+        m.plan.set_launch(B, k, 0)
+        err[k] = rel_l2(m.plan.transpose(sd, model=False).cpu().numpy().reshape(B, -1), ref)
+    print(B, {k: f"{e:.3e}" for k, e in err.items()}, flush=True)
+    assert err[-1] == err[v] <= 1.01 * err[2 if B <= 16 else 39]
+
+
 def test_one_sinogram_tile_variants_match_oracle():
     """Every one-sinogram tile form on a real arc geometry (the tile windows fit the LDS only
     for smooth travel times): forward choices 2, 3 (record streaming), 5, 6, 7 (tile form, thread
