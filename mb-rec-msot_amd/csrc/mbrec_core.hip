@@ -391,10 +391,11 @@ static int build_sir_pull(Plan *p, const std::vector<int32_t> &slot_pix, const s
     if ((size_t)p->Nsir_build * stride + 64 >= ((size_t)1 << 31) || maxlen >= (1 << 15) || p->P >= (1 << 28) ||
         span >= (1 << 15))
         return MBREC_OK;   // the packed record does not fit: the SIR forward keeps the bucketed form only
-    std::vector<float> sw((size_t)p->Nsir_build * stride + 64, 0.0f);
+    // the margins are -0 and a window's own zeros +0, so that a weight tells whether it is a tap's
+    std::vector<float> sw((size_t)p->Nsir_build * stride + 64, -0.0f);
     for (int k = 0; k < p->Nsir_build; ++k)
         for (int i = 0; i < win[2 * (size_t)k + 1]; ++i)
-            sw[(size_t)k * stride + kSirWinPad + i] = sirf[(size_t)k * Ls + win[2 * (size_t)k] + i];
+            sw[(size_t)k * stride + kSirWinPad + i] = sirf[(size_t)k * Ls + win[2 * (size_t)k] + i] + 0.0f;
     // CSR over (detector, phase m, nf): list (d, m) starts at off[(3 d + m) (n_nf + 1)]
     std::vector<int32_t> off((size_t)p->D * 3 * (n_nf + 1), 0);
     std::vector<int32_t> nfb((size_t)p->D * p->Pd, INT32_MIN);

@@ -2849,6 +2849,8 @@ __global__ __launch_bounds__(1024) void k_gather_tas(const int4 *__restrict__ st
 // sums in LDS (every pixel once per detector): FP64 with NCB = 1, and FP64 partial images, where
 // the compensated record-lane form ran before (300^2 x 8: 2.4e-7 from 64 bits, 2.6e-7 there, 2.9e-7 with
 // FP32 sums); with NCB = 2 FP32, moved to FP32 registers every eight detectors, as k_gather_tas.
+// A group's product reads all 32 samples for every pair, so where a result is not finite the pairs are
+// summed once more over their own taps (one test per group: 2 % of the stage).
 // Two workgroups share a CU, one waiting for its rows and weights while the other multiplies.
 // Bound by the matrix cores: about 18 groups of 1024 cycles (NCB = 2) per tile and detector, at
 // 400^2 x 64 2.4 of 4.4 ms; the rest is the two barriers per detector.  Gather stage against the
@@ -2969,7 +2971,7 @@ __global__ __launch_bounds__(512, 4) void k_gather_sg(const int32_t *__restrict_
             mul(0);
             // lane: sinogram i (+ 16 c), pairs 4 q + r (past the group's end: to a row that nobody reads)
             Sum *px[4], pv[4][NCB];
-            float ur[4], v[4][NCB];
+            float ur[4], v[4][NCB], chk = 0.0f;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 px[r] = s_acc + (4 * q + r < cnt ? (slc[k] >> 8 * r) & 255 : 256) * LB + i;
@@ -2983,7 +2985,34 @@ __global__ __launch_bounds__(512, 4) void k_gather_sg(const int32_t *__restrict_
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll
-                for (int c = 0; c < NCB; ++c) v[r][c] = fmaf(ur[r], acc[1][c][r] - acc[0][c][r], acc[0][c][r]);
+                for (int c = 0; c < NCB; ++c) {
+                    v[r][c] = fmaf(ur[r], acc[1][c][r] - acc[0][c][r], acc[0][c][r]);
+                    chk = fmaf(v[r][c], 0.0f, chk);
+                }
+            if (__any(chk != chk)) {
+                // an infinity or a NaN among the window's 32 samples (rare): each pair over its own taps only
+                // (the margins of the weights are -0, no tap's weight is)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int2 en = ent[(((size_t)tile * D + d) * kSgGroups + g) * 16 + 4 * q + r];
+                    const float *rr = s_row + (3 * (gh & 255) + ((gh >> 8) & 255)) * LB + i;
+                    float a0[NCB], a1[NCB];
+#pragma unroll
+                    for (int c = 0; c < NCB; ++c) a0[c] = a1[c] = 0.0f;
+#pragma unroll 1
+                    for (int t = 0; t < kSgWin; ++t, rr += 3 * LB) {
+                        const float wt = sirw[en.x + t];
+                        if (__float_as_int(wt) == (int)0x80000000) continue;
+#pragma unroll
+                        for (int c = 0; c < NCB; ++c) {
+                            a0[c] = fmaf(wt, rr[16 * c], a0[c]);
+                            a1[c] = fmaf(wt, rr[LB + 16 * c], a1[c]);
+                        }
+                    }
+#pragma unroll
+                    for (int c = 0; c < NCB; ++c) v[r][c] = fmaf(__int_as_float(en.y), a1[c] - a0[c], a0[c]);
+                }
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r)
 #pragma unroll

@@ -285,6 +285,55 @@ def test_sir_transpose_groups_match_oracle(B, crop):
     assert ran == 4      # the geometry's pairs fit the groups
 
 
+@pytest.mark.parametrize("sir", [False, True])
+@pytest.mark.parametrize("B", [4, 9, 16, 28, 64])
+def test_transpose_keeps_non_finite_samples_apart(sir, B):
+    """Infinite and NaN samples reach the pixels of their own pairs' taps only, and their own sinogram only:
+    every batch gather against the record-lane form (2), which reads a pair's own bins and no others.  The
+    SIR windows hold zeros, whose taps count."""
+    import torch
+    from mbrec.model import DevicePlan
+    _log(f"non-finite samples sir={sir} B={B}")
+    Nz, Nx, D, R, Ls = 37, 53, 9, 2.6666666666666665, 31
+    tt = geometry_tt(Nz, Nx, 1e-4, D, 0.01, 160.0, 1500.0, 4e7).reshape(D, -1)
+    tt = tt - int(tt.min()) + 10                       # some taps before the first sample
+    nT = int(tt.max()) + 5
+    g = rng(901)
+    kw = {}
+    if sir:
+        nsir = 40
+        sir_t = g.standard_normal((nsir, Ls))
+        se = np.zeros((nsir, 2), dtype=np.int32)
+        for k in range(nsir):
+            s0 = int(g.integers(3, 6))
+            se[k] = (s0, s0 + int(g.integers(14, 25)) - 1)
+            sir_t[k, s0 + 4] = 0.0
+            sir_t[k, s0 + 6] = -0.0
+        kw["sir"] = (g.integers(1, nsir + 1, size=(D, Nz * Nx)).astype(np.int32), sir_t, se)
+    plan = DevicePlan(Nz, Nx, D, nT, R, tt, **kw)
+    y = g.standard_normal((B, D, nT)).astype(np.float32)
+    for b, d, t, v in [(0, 4, nT // 2, np.inf), (1, 2, nT // 3, -np.inf), (3, 7, 2, np.nan), (B - 1, 8, nT - 3, np.inf),
+                       (B - 1, 1, nT // 4, np.nan)]:
+        y[b, d, t] = v
+    yd = torch.tensor(y).cuda()
+    plan.set_launch(B, 2, 0)
+    want = plan.transpose(yd, model=False).cpu().numpy()
+    bad = ~np.isfinite(want)
+    assert bad[[0, 1, B - 1]].any(axis=(1, 2)).all() and not bad[2].any() and bad.mean() < 0.6
+    ran = []
+    for v in range(-1, 63):
+        try:
+            plan.set_launch(B, v, 0)
+        except Exception:
+            continue
+        ran.append(v)
+        x = plan.transpose(yd, model=False).cpu().numpy()
+        assert np.array_equal(~np.isfinite(x), bad), v
+        assert rel_l2(x[~bad], want[~bad]) < TOL_OP, v
+    assert not sir or {59, 60, 61, 62}.issubset(ran)
+    assert sir or B < 9 or {55, 56, 57, 58}.issubset(ran)
+
+
 def test_default_forward_choice_can_be_set():
     """The automatic forward choice of batches of 9 to 12 is one that set_launch and the autotuner take."""
     _log("default forward choice")
