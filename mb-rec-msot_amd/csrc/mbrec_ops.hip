@@ -1863,33 +1863,41 @@ __global__ __launch_bounds__(256) void k_fwd_sir_pull_bl(const int4 *__restrict_
 // records whose weight matrix has the records' windows as columns.  A wave takes a run of rb
 // bands of nfb first samples; the records of a band [a, a + nfb) have their taps (and the
 // u-part of phase 2, one sample on) on the 32 samples from a.  Two records per product
-// 32x32x2: A = 32 weights of each from the zero-margin table (one 128-byte run per record)
-// times 1 - u or u, B = the records' pixel rows (32 sinograms).  Every record is visited once,
-// for 32 NC sinograms at a time; the accumulators are the samples' three bins.
+// 32x32x2: A = 32 weights of each from the zero-margin table (one 128-byte run per record),
+// B = the records' pixel rows (32 sinograms) times 1 - u or u.  Every record is visited once,
+// for 32 sinograms at a time; the accumulators are the samples' three bins.
 // With nfb = 8 (windows of at most 24 taps) the next band's samples are the same accumulators
 // eight rows on -- four registers of the 32x32 layout -- so a band's first eight samples
 // leave for the band scratch and the rest moves up (registers only); a run ends with 24 rows
 // that the next run adds to (rb = 1: all 32 rows leave, any nfb <= 32 - longest window).
 // Taps on samples outside [0, span) have their weights masked (the reference's range check).
 // Pass 2 adds the overlapping rows in run order.
+// Sums: 128 records of a phase at a time, added to the run's accumulators (one chain over all a run's
+// records had twice the error, 2.1e-6 from the model operator in 64 bits at 200^2 against 1.45e-6, and
+// that of the vector form before it 2.05e-6; adding up 64 at a time: 1.3e-6, 5 % slower).
 // Bound by the matrix cores: 2 products of 64 cycles per two records and 32 sinograms (at
-// 400^2 and 64 sinograms 2.1 ms of matrix time); without any loads the loop still takes 0.9 of
-// its 1.2 ms at 300^2 x 28 (0.6 ms of matrix time).  Forward operator against the vector form
-// that issued 60 FMAs per record and 64 lanes: 300^2 x 28 4.98 -> 1.49 ms, 400^2 x 64
-// 8.88 -> 4.02 ms, 300^2 x 2 4.86 -> 1.3 ms.  Four bands per run: the scratch is 1.75 rows per
+// 400^2 and 64 sinograms 2.1 ms of matrix time), two waves per SIMD (148 registers).  Forward stage against
+// the vector form that issued 60 FMAs per record and 64 lanes: 300^2 x 28 4.75 -> 1.35 ms, 400^2 x 64
+// 8.4 -> 4.4 ms, 300^2 x 4 4.55 -> 1.23 ms.  Four bands per run: the scratch is 1.75 rows per
 // sample, and one wave per workgroup keeps the last waves short (eight bands: 0.2 ms more).
-// 64 sinograms per wave read each weight once for both halves (two waves of 32: 8 % more).
+// Waves of 64 sinograms, which read each weight once for both halves, hold 256 registers and one wave
+// per SIMD: no faster (4.3 to 4.6 ms).
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kSirRunTail = 24;   // rows of a run (rb > 1) past its own first samples
 
-template <int NC, int M>
-__device__ __forceinline__ void sir_mf_phase(f32x16 (&acc)[3][NC], const int4 *__restrict__ rec, int rs, int re,
+template <int M>
+__device__ __forceinline__ void sir_mf_phase(f32x16 (&acc)[3], const int4 *__restrict__ rec, int rs, int re,
                                              const float *__restrict__ imgI, const float *__restrict__ sirw, int a,
-                                             int span, int zoff, int Bp, const int (&col)[NC])
+                                             int span, int zoff, int Bp, int col)
 {
     constexpr int U = 8;   // products whose operands are in flight while the previous U run
     const int lane = threadIdx.x & 63, t = lane & 31, hl = lane >> 5;
     const bool in0 = a + t >= 0 && a + t < span, in1 = a + t >= 1 && a + t <= span;   // sample, sample before
+    f32x16 s[2];   // up to 128 records' sums
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[j][i] = 0.0f;
     int4 e = rec[max(min(rs + lane, re - 1), 0)];
     for (int c0 = rs; c0 < re; c0 += 64) {
         // lane = record; past the end: the last record with zero weights
@@ -1897,32 +1905,24 @@ __device__ __forceinline__ void sir_mf_phase(f32x16 (&acc)[3][NC], const int4 *_
         const float u = __int_as_float(e.z);
         const int nk = min(32, (re - c0 + 1) / 2);
         e = rec[max(min(c0 + 64 + lane, re - 1), 0)];   // the next 64, in flight during these
-        float A0[2][U], A1[2][U], uu[2][U], Bv[2][U][NC];
-        auto load = [&](int k, int s) __attribute__((always_inline)) {
+        float A0[2][U], A1[2][U], uu[2][U], Bv[2][U];
+        auto load = [&](int k, int h) __attribute__((always_inline)) {
 #pragma unroll
             for (int q = 0; q < U; ++q) {
                 const int src = min(2 * (k + q) + hl, 63);
                 const float *w = sirw + __shfl(wo, src) + t;
-                A0[s][q] = w[0];
-                A1[s][q] = M == 2 ? w[-1] : 0.0f;
-                uu[s][q] = __shfl(u, src);
-                const float *row = imgI + (size_t)__shfl(px, src) * Bp;
-#pragma unroll
-                for (int n = 0; n < NC; ++n) Bv[s][q][n] = row[col[n]];
+                A0[h][q] = w[0];
+                A1[h][q] = M == 2 ? w[-1] : 0.0f;
+                uu[h][q] = __shfl(u, src);
+                Bv[h][q] = imgI[(size_t)__shfl(px, src) * Bp + col];
             }
         };
-        auto mul = [&](int s) __attribute__((always_inline)) {
+        auto mul = [&](int h) __attribute__((always_inline)) {
 #pragma unroll
             for (int q = 0; q < U; ++q) {
-                const float w0 = in0 ? A0[s][q] : 0.0f, w1 = M == 2 ? (in1 ? A1[s][q] : 0.0f) : w0;
-                const float f0 = w0 * (1.0f - uu[s][q]), f1 = w1 * uu[s][q];
-#pragma unroll
-                for (int n = 0; n < NC; ++n)
-                    acc[M][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(f0, Bv[s][q][n], acc[M][n], 0, 0, 0);
-#pragma unroll
-                for (int n = 0; n < NC; ++n)
-                    acc[(M + 1) % 3][n] =
-                        __builtin_amdgcn_mfma_f32_32x32x2f32(f1, Bv[s][q][n], acc[(M + 1) % 3][n], 0, 0, 0);
+                const float w0 = in0 ? A0[h][q] : 0.0f, w1 = M == 2 ? (in1 ? A1[h][q] : 0.0f) : w0;
+                s[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(w0, Bv[h][q] * (1.0f - uu[h][q]), s[0], 0, 0, 0);
+                s[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(w1, Bv[h][q] * uu[h][q], s[1], 0, 0, 0);
             }
         };
         load(0, 0);
@@ -1938,10 +1938,18 @@ __device__ __forceinline__ void sir_mf_phase(f32x16 (&acc)[3][NC], const int4 *_
             mul(1);
             __builtin_amdgcn_sched_barrier(0);
         }
+        if (((c0 - rs) & 64) || c0 + 64 >= re) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    acc[(M + j) % 3][i] += s[j][i];
+                    s[j][i] = 0.0f;
+                }
+        }
     }
 }
 
-template <int NC>
 __global__ __launch_bounds__(64) void k_fwd_sir_band(const int4 *__restrict__ rec, const int32_t *__restrict__ off,
                                                       const float *__restrict__ imgI, const float *__restrict__ sirw,
                                                       float *__restrict__ scratch, int D, int span, int lo, int n_nf,
@@ -1949,28 +1957,22 @@ __global__ __launch_bounds__(64) void k_fwd_sir_band(const int4 *__restrict__ re
 {
     const int lane = threadIdx.x & 63, j = lane & 31;
     const int run = blockIdx.x / D, d = blockIdx.x - run * D;
-    const int b0 = blockIdx.y * 32 * NC;
-    int a = lo + run * nfb * rb, col[NC];
-#pragma unroll
-    for (int n = 0; n < NC; ++n) col[n] = min(b0 + 32 * n + j, Bp - 1);
+    const int b0 = blockIdx.y * 32, col = min(b0 + j, Bp - 1);
+    int a = lo + run * nfb * rb;
     const int rows = rb > 1 ? 8 * rb + kSirRunTail : 32;
     float *dst = scratch + ((size_t)d * nrun + run) * rows * 3 * Bp + b0 + j + (size_t)(4 * (lane >> 5)) * 3 * Bp;
-    f32x16 acc[3][NC];
+    f32x16 acc[3];
 #pragma unroll
     for (int m = 0; m < 3; ++m)
 #pragma unroll
-        for (int n = 0; n < NC; ++n)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[m][n][i] = 0.0f;
+        for (int i = 0; i < 16; ++i) acc[m][i] = 0.0f;
     // rows 8 g + 4 (lane / 32) + i of the accumulators (register 4 g + i) to row r0 + ...
     auto store = [&](int g, int r0) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int m = 0; m < 3; ++m)
-#pragma unroll
-                for (int n = 0; n < NC; ++n)
-                    if (b0 + 32 * n + j < Bp) dst[((size_t)(r0 + i) * 3 + m) * Bp + 32 * n] = acc[m][n][4 * g + i];
+                if (b0 + j < Bp) dst[((size_t)(r0 + i) * 3 + m) * Bp] = acc[m][4 * g + i];
     };
     const int32_t *o = off + (size_t)d * 3 * (n_nf + 1);
     for (int band = 0; band < rb; ++band, a += nfb) {
@@ -1979,15 +1981,13 @@ __global__ __launch_bounds__(64) void k_fwd_sir_band(const int4 *__restrict__ re
 #pragma unroll
             for (int m = 0; m < 3; ++m)
 #pragma unroll
-                for (int n = 0; n < NC; ++n)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[m][n][i] = i < 12 ? acc[m][n][(i + 4) & 15] : 0.0f;
+                for (int i = 0; i < 16; ++i) acc[m][i] = i < 12 ? acc[m][(i + 4) & 15] : 0.0f;
         }
         const int ia = a - lo, ib = min(ia + nfb, n_nf);
         if (ia >= n_nf) continue;
-        sir_mf_phase<NC, 0>(acc, rec, o[ia], o[ib], imgI, sirw, a, span, zoff, Bp, col);
-        sir_mf_phase<NC, 1>(acc, rec, o[n_nf + 1 + ia], o[n_nf + 1 + ib], imgI, sirw, a, span, zoff, Bp, col);
-        sir_mf_phase<NC, 2>(acc, rec, o[2 * (n_nf + 1) + ia], o[2 * (n_nf + 1) + ib], imgI, sirw, a, span, zoff, Bp, col);
+        sir_mf_phase<0>(acc, rec, o[ia], o[ib], imgI, sirw, a, span, zoff, Bp, col);
+        sir_mf_phase<1>(acc, rec, o[n_nf + 1 + ia], o[n_nf + 1 + ib], imgI, sirw, a, span, zoff, Bp, col);
+        sir_mf_phase<2>(acc, rec, o[2 * (n_nf + 1) + ia], o[2 * (n_nf + 1) + ib], imgI, sirw, a, span, zoff, Bp, col);
     }
 #pragma unroll
     for (int g = 0; g < 4; ++g) store(g, 8 * (rb - 1) + 8 * g);
@@ -3943,12 +3943,6 @@ static int launch_scatter(Plan *p, const float *imgI, int B, int Bp, hipStream_t
             const int step = p->sband_nfb * p->sband_rb;
             const int zoff = p->sirw_zero + 1;   // zeros from one before to 31 after
             const unsigned nwg = (unsigned)((p->sband_nrun + 7) / 8 * 8 * ((p->D + 3) / 4));
-            // 64 sinograms per wave where a part of the second half is used, else 32
-            const auto launch = [&](auto kern, int nc) {
-                hipLaunchKernelGGL(kern, dim3(p->sband_nrun * p->D, (Bp + 32 * nc - 1) / (32 * nc)), dim3(64), 0, s,
-                                   p->d_srec, p->d_srec_off, imgI, p->d_sirw, p->d_sband, p->D, span, p->sp_lo, p->sp_n,
-                                   p->sband_nfb, p->sband_rb, p->sband_nrun, zoff, Bp);
-            };
             const auto sum = [&](auto kern, int v) {
                 hipLaunchKernelGGL(kern, dim3((unsigned)(((size_t)p->geom.NB * Bp / v + 255) / 256), p->D), dim3(256), 0, s,
                                    (const float *)p->d_sband, p->d_bins, p->geom.NB, p->sp_lo, step,
@@ -3958,8 +3952,10 @@ static int launch_scatter(Plan *p, const float *imgI, int B, int Bp, hipStream_t
                 hipLaunchKernelGGL(k_fwd_sir_band1, dim3(nwg), dim3(256), 0, s, p->d_srec, p->d_srec_off, imgI,
                                    p->d_sirw, p->d_sband, p->D, span, p->sp_lo, p->sp_n, p->sband_nfb, p->sband_rb,
                                    p->sband_nrun, zoff);
-            else if (Bp > 32) launch(k_fwd_sir_band<2>, 2);
-            else launch(k_fwd_sir_band<1>, 1);
+            else
+                hipLaunchKernelGGL(k_fwd_sir_band, dim3(p->sband_nrun * p->D, (Bp + 31) / 32), dim3(64), 0, s, p->d_srec,
+                                   p->d_srec_off, imgI, p->d_sirw, p->d_sband, p->D, span, p->sp_lo, p->sp_n,
+                                   p->sband_nfb, p->sband_rb, p->sband_nrun, zoff, Bp);
             if (Bp == 1) sum(k_fwd_sir_band_sum<1>, 1);
             else sum(k_fwd_sir_band_sum<4>, 4);
         } else if (Bp == 1) {

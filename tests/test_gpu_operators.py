@@ -468,6 +468,30 @@ def test_sir_batch_gather_sums_as_close_as_before(B, v):
     assert err[-1] == err[v] <= 1.01 * err[2 if B <= 16 else 39]
 
 
+@pytest.mark.parametrize("B", [2, 28, 64])
+def test_sir_forward_sums_as_close_as_before(B):
+    """The matrix-core SIR forward adds up 200 x 200 pixels of one sign: its distance to the FP64 oracle is no
+    larger than that of the vector pull form (1000), which sums a sample's records one by one as the form
+    before it did."""
+    import torch
+    _log(f"SIR forward sums B={B}")
+    D, nT, n = 6, 1000, 200
+    m = _geometry_model(n, n, D, nT, 1e-4, sir=True, sigma=1.0)
+    tt, d = _oracle_of(m).tt.T, m.Data
+    g = rng(38)
+    c, r2 = g.uniform(0, n, (2, B, 1, 1)), ((np.arange(n)[:, None], np.arange(n)[None, :]))
+    x = (0.5 + g.uniform(0, 1, (B, 1, 1)) * ((r2[0] - c[0]) ** 2 + (r2[1] - c[1]) ** 2 < 50.0 ** 2)).astype(np.float32)
+    ref = np.transpose(O.forward_sir(x.reshape(B, -1), d.SPMRIndices.reshape(D, -1).T, tt, d.SPMR.T, nT,
+                                     d.SPMRTimestepIndexStartAndEnd.T, _oracle_of(m).R), (0, 2, 1))
+    xd = torch.tensor(x, dtype=torch.float32).cuda()
+    err = {}
+    for k in (0, 1004, 1000):
+        m.plan.set_launch(B, -1, k)
+        err[k] = rel_l2(m.plan.forward(xd, model=False).cpu().numpy(), ref)
+    print(B, {k: f"{e:.3e}" for k, e in err.items()}, flush=True)
+    assert err[0] == err[1004] <= err[1000]
+
+
 def test_one_sinogram_tile_variants_match_oracle():
     """Every one-sinogram tile form on a real arc geometry (the tile windows fit the LDS only
     for smooth travel times): forward choices 2, 3 (record streaming), 5, 6, 7 (tile form, thread
