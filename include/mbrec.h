@@ -131,7 +131,8 @@ int mbrec_plan_autotune(mbrec_plan plan, int B, int reps, mbrec_stream s, int *c
  * there, or lane groups of samples for windows of more than 31 taps; batches: 24 samples x 2
  * records in flight per wave), 1001 / 1002 / 1003 batch pull forms with (16, 4), (16, 2),
  * (32, 1), 1004 the band form for batches on the matrix cores (each record once, overlapping
- * rows summed in a second pass; the default for batches);
+ * rows summed in a second pass; the default for batches with windows of at most 31 taps, 30
+ * above 32 sinograms);
  * bucketed scatter: > 0 the
  * record-lane kernel with that LDS batch chunk (a multiple of 4), < 0 the
  * batch-lane kernel with lane groups of -value (16, 32 or 64) sinograms.  Plans

@@ -61,7 +61,7 @@ static void free_work(Plan *p)
         if (q) (void)hipFree(q);
     p->d_bins = p->d_hpart = p->d_imgI = p->d_img_tmp = p->d_sino_tmp = p->d_gpart = p->d_sband = nullptr;
     p->d_img_slot = nullptr;
-    p->sband_nrun = p->sband_nfb = p->sband_rb = 0;
+    p->sband_nrun = p->sband_nfb = p->sband_rb = p->sband_cols = 0;
     p->bcap = 0;
     p->work_bytes = 0;
 }
@@ -138,18 +138,21 @@ int ensure_work(Plan *p, int B)
         free_work(p);
         return rc;
     }
-    // band-form SIR forward rows: a band's taps and the sample after them stay within 32 samples
+    // band-form SIR forward rows: a band's taps and the sample after them stay within 32 samples.  Windows of
+    // 31 taps leave one first sample per band and 32 rows for each (400^2 x 64: 12.9 GB): 200^2 x 64 took 5.9 ms
+    // against 3.7 ms of the pull form (x 28 2.8 / 3.5 ms), which larger batches than 32 then keep
     if (p->use_sir && p->d_srec && p->sir_maxlen < kSirBandTS) {
         const int nfb = p->sir_maxlen <= kSirBandTS - kSirBandShift ? kSirBandShift : kSirBandTS - p->sir_maxlen;
         const int rb = nfb == kSirBandShift ? kSirBandRun : 1;
         const int nrun = (p->sp_n + nfb * rb - 1) / (nfb * rb);
-        if ((rc = dalloc(&p->d_sband, (size_t)p->D * nrun * sband_rows(rb) * 3 * Bp, &acc))) {
-            free_work(p);
-            return rc;
+        const int cols = nfb > 1 ? Bp : std::min(Bp, 32);
+        // without memory for the rows the pull forms run
+        if (dalloc(&p->d_sband, (size_t)p->D * nrun * sband_rows(rb) * 3 * cols, &acc) == MBREC_OK) {
+            p->sband_cols = cols;
+            p->sband_nrun = nrun;
+            p->sband_nfb = nfb;
+            p->sband_rb = rb;
         }
-        p->sband_nrun = nrun;
-        p->sband_nfb = nfb;
-        p->sband_rb = rb;
     }
     // the two zero rows after the last detector's bins (pairs outside the bin range read them)
     MBREC_HIP(hipMemset(p->d_bins + (size_t)p->D * p->geom.NB * Bp, 0, sizeof(float) * 2 * Bp));

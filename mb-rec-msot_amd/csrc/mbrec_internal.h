@@ -170,8 +170,8 @@ struct Plan {
     float *d_sino_tmp = nullptr; // [B][D][nT]       samples before/after the IR filter
     float *d_gpart = nullptr;    // [max(8 B, 16)][P]  partial images of the detector-grouped gathers
     float *d_img_slot = nullptr; // [Pd]  one sinogram's image in slot order (pull forward)
-    float *d_sband = nullptr;    // [D][runs][rows][3][Bp]  band-form SIR forward rows
-    int sband_nrun = 0, sband_nfb = 0, sband_rb = 0;
+    float *d_sband = nullptr;    // [D][runs][rows][3][Bp]  band-form SIR forward rows, Bp <= sband_cols
+    int sband_nrun = 0, sband_nfb = 0, sband_rb = 0, sband_cols = 0;
     int sirw_zero = 0;           // first of 64 zeros at the end of d_sirw
     size_t table_bytes = 0;
     size_t work_bytes = 0;

@@ -3332,11 +3332,10 @@ constexpr int kSirPull = 1000, kSirPullVariants = 5, kSirBand = kSirPull + 4;
 
 static bool is_sir_pull(int c) { return c >= kSirPull && c < kSirPull + kSirPullVariants; }
 
-// tables and scratch of the band form are there (windows of at most 31 taps)
+// tables and scratch of the band form are there (windows of at most 31 taps, 30 above 32 sinograms)
 static bool sir_band_ok(const Plan *p, int Bp)
 {
-    return p->use_sir && p->d_srec && p->d_sirw && p->d_sband && p->sband_nfb >= 1 && p->bcap >= 1 &&
-           batch_stride(p->bcap) >= Bp;
+    return p->use_sir && p->d_srec && p->d_sirw && p->d_sband && p->sband_nfb >= 1 && p->sband_cols >= Bp;
 }
 
 static bool sir_pull_ok(const Plan *p, int Bp, int c = kSirPull)

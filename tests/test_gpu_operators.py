@@ -213,7 +213,7 @@ def test_every_launch_variant_matches_oracle(sir, B):
 
 
 @pytest.mark.parametrize("length,B", [(1, 1), (24, 1), (25, 1), (31, 1), (32, 1), (24, 2), (25, 33), (31, 32), (32, 4),
-                                      (8, 64), (24, 67)])
+                                      (8, 64), (24, 67), (30, 33), (31, 33)])
 def test_sir_forward_band_edges(length, B):
     """The band forms of the SIR forward at the window lengths where they change (24: bands that
     slide, 31: longest window of a band, 32: the forms without bands) and at the edges of a
@@ -241,6 +241,19 @@ def test_sir_forward_band_edges(length, B):
     y = plan.forward(torch.tensor(x, dtype=torch.float32).cuda(), model=False).cpu().numpy()
     assert rel_l2(y, yo) < TOL_OP
     assert np.abs(y - yo).max() < 1e-4 * np.abs(yo).max()
+    if B == 1:
+        return
+    # the band form is there up to 31 taps, up to 30 above 32 sinograms, and whatever the workspace held before
+    has_band = length < (31 if B > 32 else 32)
+    for _ in range(2):
+        if has_band:
+            plan.set_launch(B, -1, 1004)
+            assert np.array_equal(plan.forward(torch.tensor(x, dtype=torch.float32).cuda(), model=False).cpu().numpy(), y)
+        else:
+            with pytest.raises(Exception):
+                plan.set_launch(B, -1, 1004)
+        plan.set_launch(B, -1, 0)
+        plan.forward(torch.zeros((70, Nx, Nz), device="cuda"), model=False)
 
 
 @pytest.mark.parametrize("B", [2, 4, 13, 16, 17, 28, 33, 70])
