@@ -5,8 +5,10 @@
 #include <cstdarg>
 #include <cstdio>
 #include <atomic>
+#include <memory>
 #include <mutex>
 #include <cstring>
+#include <exception>
 #include <system_error>
 #include <thread>
 #include <vector>
@@ -111,8 +113,11 @@ hipError_t device_malloc(void **p, size_t bytes)
     return hipMalloc(p, bytes);
 }
 
+static void ensure_sir_groups(Plan *p);
+
 int ensure_work(Plan *p, int B)
 {
+    if (p->use_sir && batch_stride(B) >= 4) ensure_sir_groups(p);
     const size_t need_h = std::max<size_t>((size_t)p->D * p->nbk * p->WL, 1);
     if (B <= p->bcap && p->d_hpart && p->work_bytes && need_h * batch_stride(p->bcap) * sizeof(float) <=
                                                              p->work_bytes)
@@ -554,11 +559,10 @@ static int build_sir_tiles(Plan *p, const std::vector<int32_t> &slot_pix, const 
 // the range check is the window's (a pair's offset points at its weight on the window's first
 // sample: the zero margins of d_sirw give the rest).  No tables where a (tile, detector) needs more
 // than 24 groups or 256 rows, or the axis is shorter than a window.
-static int build_sir_groups(Plan *p, const std::vector<int32_t> &slot_pix, const std::vector<int32_t> &tq,
-                            const int32_t *sidx, const int32_t *win, int Ls)
+// Built at a plan's first batch (3.5 KB per (tile, detector): 0.57 GB at 400^2 x 256, and as much on the
+// host meanwhile), from the plan's own tables; where memory runs out the other SIR forms run.
+static void free_sir_groups(Plan *p)
 {
-    const BinGeom &g = p->geom;
-    const int span = g.nT + 2 * g.K, half = Ls / 2, ntile = p->Pd / 256;
     for (void *q : {(void *)p->d_sghdr, (void *)p->d_sgent, (void *)p->d_sgslot})
         if (q) (void)hipFree(q);
     p->table_bytes -= p->sg_bytes;
@@ -567,14 +571,27 @@ static int build_sir_groups(Plan *p, const std::vector<int32_t> &slot_pix, const
     p->d_sgent = nullptr;
     p->d_sgslot = nullptr;
     p->sg_rows = 0;
-    int maxlen = 0;
-    for (int k = 0; k < p->Nsir_build; ++k) maxlen = std::max(maxlen, (int)win[2 * (size_t)k + 1]);
+    p->sg_tried = false;
+}
+
+static int build_sir_groups(Plan *p)
+{
+    const BinGeom &g = p->geom;
+    const int span = g.nT + 2 * g.K, half = p->Ls / 2, ntile = p->Pd / 256;
+    const int maxlen = p->sir_maxlen;
     if (!p->d_sirw || maxlen > kSgWin || span < kSgWin) return MBREC_OK;
+    std::vector<int32_t> slot_pix(p->Pd), tq((size_t)p->D * p->Pd), sidx(tq.size()), win(2 * (size_t)p->Nsir);
+    MBREC_HIP(hipMemcpy(slot_pix.data(), p->d_pix, sizeof(int32_t) * slot_pix.size(), hipMemcpyDeviceToHost));
+    MBREC_HIP(hipMemcpy(tq.data(), p->d_tq, sizeof(int32_t) * tq.size(), hipMemcpyDeviceToHost));
+    MBREC_HIP(hipMemcpy(sidx.data(), p->d_sidx, sizeof(int32_t) * sidx.size(), hipMemcpyDeviceToHost));
+    MBREC_HIP(hipMemcpy(win.data(), p->d_swin, sizeof(int32_t) * win.size(), hipMemcpyDeviceToHost));
     const int stride = maxlen + 2 * kSirWinPad;
     const size_t ntd = (size_t)ntile * p->D;
+    // zeroed tile by tile by the threads below
+    const size_t nent = ntd * kSgGroups * 16, nslot = ntd * kSgGroups * 4;
     std::vector<int32_t> hdr(ntd * 32, 0);
-    std::vector<int2> ent(ntd * kSgGroups * 16, make_int2(0, 0));
-    std::vector<uint32_t> slot(ntd * kSgGroups * 4, 0u);
+    const std::unique_ptr<int2[]> ent(new int2[nent]);
+    const std::unique_ptr<uint32_t[]> slot(new uint32_t[nslot]);
     const float scale = std::ldexp(1.0f, -g.F);
     std::atomic<bool> fits{true};
     std::atomic<int> ns_max{0};
@@ -584,6 +601,9 @@ static int build_sir_groups(Plan *p, const std::vector<int32_t> &slot_pix, const
             float u;
         };
         Pair pr[256];
+        const size_t per = (size_t)p->D * kSgGroups;
+        std::fill_n(ent.get() + t * per * 16, per * 16, make_int2(0, 0));
+        std::fill_n(slot.get() + t * per * 4, per * 4, 0u);
         for (int d = 0; d < p->D && fits; ++d) {
             int np = 0, lo = INT32_MAX, hi = 0;
             for (int k = 0; k < 256; ++k) {
@@ -638,13 +658,28 @@ static int build_sir_groups(Plan *p, const std::vector<int32_t> &slot_pix, const
     const int rows = 64 * ((3 * ns_max + 1 + 63) / 64);
     if (!fits || rows > 256 || !ns_max) return MBREC_OK;
     int rc;
-    if ((rc = dalloc(&p->d_sghdr, hdr.size(), &p->sg_bytes)) || (rc = dalloc(&p->d_sgent, ent.size(), &p->sg_bytes)) ||
-        (rc = dalloc(&p->d_sgslot, slot.size(), &p->sg_bytes)) || (rc = upload(p->d_sghdr, hdr.data(), hdr.size())) ||
-        (rc = upload(p->d_sgent, ent.data(), ent.size())) || (rc = upload(p->d_sgslot, slot.data(), slot.size())))
+    if ((rc = dalloc(&p->d_sghdr, hdr.size(), &p->sg_bytes)) || (rc = dalloc(&p->d_sgent, nent, &p->sg_bytes)) ||
+        (rc = dalloc(&p->d_sgslot, nslot, &p->sg_bytes)) || (rc = upload(p->d_sghdr, hdr.data(), hdr.size())) ||
+        (rc = upload(p->d_sgent, ent.get(), nent)) || (rc = upload(p->d_sgslot, slot.get(), nslot)))
         return rc;
     p->table_bytes += p->sg_bytes;
     p->sg_rows = rows;
     return MBREC_OK;
+}
+
+static void ensure_sir_groups(Plan *p)
+{
+    if (p->sg_tried) return;
+    bool ok = false;
+    try {
+        ok = build_sir_groups(p) == MBREC_OK;
+    } catch (const std::exception &) {   // no host memory
+    }
+    if (!ok) {
+        p->table_bytes += p->sg_bytes;   // counted as the finished tables are
+        free_sir_groups(p);
+    }
+    p->sg_tried = true;
 }
 
 int build_records(Plan *p, const std::vector<int32_t> &slot_pix, const std::vector<int32_t> &tq,
@@ -1058,6 +1093,7 @@ int mbrec_plan_set_sir(mbrec_plan h, const int32_t *sirIdx, const double *sir, i
     }
     p->tune = TuneChoice();
     p->use_sir = 0;
+    free_sir_groups(p);
     if (p->d_sidx) { (void)hipFree(p->d_sidx); (void)hipFree(p->d_sir); (void)hipFree(p->d_swin); }
     int rc;
     if ((rc = dalloc(&p->d_sidx, sidx.size(), &p->table_bytes)) ||
@@ -1085,7 +1121,6 @@ int mbrec_plan_set_sir(mbrec_plan h, const int32_t *sirIdx, const double *sir, i
         p->Nsir_build = Nsir;
         if ((rc = build_sir_pull(p, slot_pix, tq, sidx.data(), win.data(), Ls, sirf.data()))) return rc;
         if ((rc = build_sir_tiles(p, slot_pix, tq, sidx.data(), win.data(), Ls))) return rc;
-        if ((rc = build_sir_groups(p, slot_pix, tq, sidx.data(), win.data(), Ls))) return rc;
     }
     p->use_sir = 1;
     p->Ls = Ls;

@@ -298,6 +298,31 @@ def test_sir_transpose_groups_match_oracle(B, crop):
     assert ran == 4      # the geometry's pairs fit the groups
 
 
+def test_sir_group_tables_come_with_the_first_batch():
+    """The tables of the matrix-core SIR transpose (3.5 KB per 256-pixel tile and detector) are built for the
+    first batch: a plan used for one sinogram does without.  New SIR tables rebuild them."""
+    import torch
+    _log("SIR group tables")
+    D, nT = 64, 1000
+    m = _geometry_model(200, 200, D, nT, 1e-4, sir=True, sigma=1.0)
+    groups = 13 * 13 * D * 3584
+    sg = torch.tensor(rng(39).standard_normal((4, D, nT)), dtype=torch.float32).cuda()
+    torch.cuda.synchronize()
+
+    def used(B):
+        before = torch.cuda.mem_get_info()[0]
+        m.plan.transpose(sg[:B].contiguous(), model=False)
+        torch.cuda.synchronize()
+        return before - torch.cuda.mem_get_info()[0]
+    assert used(1) < groups
+    assert used(4) > groups
+    x = m.plan.transpose(sg, model=False).cpu().numpy()
+    d = m.Data
+    m.plan.set_sir(d.SPMRIndices.reshape(D, -1), d.SPMR, d.SPMRTimestepIndexStartAndEnd)
+    m.plan.set_launch(4, 61, 0)
+    assert np.array_equal(m.plan.transpose(sg, model=False).cpu().numpy(), x)
+
+
 @pytest.mark.parametrize("sir", [False, True])
 @pytest.mark.parametrize("B", [4, 9, 16, 28, 64])
 def test_transpose_keeps_non_finite_samples_apart(sir, B):
