@@ -9,7 +9,6 @@
 #include <mutex>
 #include <cstring>
 #include <exception>
-#include <system_error>
 #include <thread>
 #include <vector>
 #include <algorithm>
@@ -473,7 +472,7 @@ static void parallel_for(int n, F &&f)
     std::vector<std::thread> th;
     try {
         for (int k = 1; k < nt; ++k) th.emplace_back(work);
-    } catch (const std::system_error &) {   // fewer threads than asked for: the ones there do it all
+    } catch (const std::exception &) {   // fewer threads than asked for (or no memory for more): the ones there do it all
     }
     work();
     for (auto &t : th) t.join();
