@@ -239,7 +239,12 @@ def test_unet_adam_steps_reduce_loss(require_gpu):
     (3, 15, 31, 32, 32, 0, 0),      # one short of a tile in both directions, images joined inside a fragment
     (2, 16, 30, 64, 96, 1, 0),      # whole rows of tiles, images meeting at a fragment's end; 32-channel tiles
     (2, 17, 33, 96, 64, 0, 0),      # one past a tile in both directions
+    (2, 7, 63, 64, 64, 1, 0),       # the same at the edges of one tile's 8 rows
+    (1, 8, 64, 32, 128, 0, 0),
+    (3, 9, 34, 32, 64, 1, 0),
     (70, 3, 2, 32, 64, 1, 0),       # images much narrower than a fragment
+    (42, 200, 101, 192, 64, 1, 0),  # 64 output channels per workgroup: 192 channels in, over 4096 workgroups
+    (32, 200, 67, 224, 128, 0, 0),
     (1, 20, 37, 32, 32, 1, 1),      # arrays off the 16-byte alignment
 ])
 def test_conv3x3_bf16_tile_edges(require_gpu, N, H, W, Cin, Cout, relu, shift):
