@@ -1327,18 +1327,26 @@ int mbrec_conv3x3_bf16(const uint16_t *x, const uint16_t *w, const float *bias, 
     hipStream_t s = (hipStream_t)stream;
     if (!relu && bias) return set_error(MBREC_ERR_ARG, "mbrec:args", "conv3x3_bf16: bias requires relu=1");
     const size_t nx = (size_t)N * H * W * Cin * 2, nw = (size_t)Cout * 9 * Cin * 2, ny = (size_t)N * H * W * Cout * 2;
-    void *cx = nullptr, *cw = nullptr, *cy = nullptr;
+    struct Copies {
+        hipStream_t s;
+        void *x = nullptr, *w = nullptr, *y = nullptr;
+        ~Copies()
+        {
+            for (void *q : {x, w, y})
+                if (q) (void)hipFreeAsync(q, s);
+        }
+    } c{s};
     if ((uintptr_t)x % 16) {
-        MBREC_HIP(hipMallocAsync(&cx, nx, s));
-        MBREC_HIP(hipMemcpyAsync(cx, x, nx, hipMemcpyDeviceToDevice, s));
+        MBREC_HIP(hipMallocAsync(&c.x, nx, s));
+        MBREC_HIP(hipMemcpyAsync(c.x, x, nx, hipMemcpyDeviceToDevice, s));
     }
     if ((uintptr_t)w % 16) {
-        MBREC_HIP(hipMallocAsync(&cw, nw, s));
-        MBREC_HIP(hipMemcpyAsync(cw, w, nw, hipMemcpyDeviceToDevice, s));
+        MBREC_HIP(hipMallocAsync(&c.w, nw, s));
+        MBREC_HIP(hipMemcpyAsync(c.w, w, nw, hipMemcpyDeviceToDevice, s));
     }
-    if ((uintptr_t)y % 8) MBREC_HIP(hipMallocAsync(&cy, ny, s));
-    const Feat fx{cx ? (uint16_t *)cx : const_cast<uint16_t *>(x), Cin}, fy{cy ? (uint16_t *)cy : y, Cout};
-    const uint16_t *fw = cw ? (const uint16_t *)cw : w;
+    if ((uintptr_t)y % 8) MBREC_HIP(hipMallocAsync(&c.y, ny, s));
+    const Feat fx{c.x ? (uint16_t *)c.x : const_cast<uint16_t *>(x), Cin}, fy{c.y ? (uint16_t *)c.y : y, Cout};
+    const uint16_t *fw = c.w ? (const uint16_t *)c.w : w;
     ConvArgs a = conv_args(whole(fx), Cin, fw, Cout, N, H, W);
     a.y = fy.p;
     a.ys = Cout;
@@ -1346,10 +1354,8 @@ int mbrec_conv3x3_bf16(const uint16_t *x, const uint16_t *w, const float *bias, 
     const bool far = nx / 16 >= (size_t)INT32_MAX;   // slots beyond 32-bit indices
     if (relu) far ? conv_launch<kRelu, long long>(a, s) : conv_launch<kRelu>(a, s);
     else far ? conv_launch<kGrad, long long>(a, s) : conv_launch<kGrad>(a, s);   // plain convolution
-    if (cy) MBREC_HIP(hipMemcpyAsync(y, cy, ny, hipMemcpyDeviceToDevice, s));
-    for (void *q : {cx, cw, cy})
-        if (q) MBREC_HIP(hipFreeAsync(q, s));
     MBREC_HIP(hipGetLastError());
+    if (c.y) MBREC_HIP(hipMemcpyAsync(y, c.y, ny, hipMemcpyDeviceToDevice, s));
     return MBREC_OK;
 }
 
