@@ -530,6 +530,61 @@ def test_sir_forward_sums_as_close_as_before(B):
     assert err[0] == err[1004] <= err[1000]
 
 
+@pytest.mark.parametrize("B", [13, 16, 28, 33, 64])
+def test_lds_gather_many_detectors_match_oracle(B):
+    """The LDS gathers of batches without SIR with more than eight detectors in a group and a last group that
+    is shorter (75 detectors in groups of 38 and 19): all four forms are valid on this geometry, one of them is
+    the automatic choice."""
+    import torch
+    _log(f"LDS gather 75 detectors B={B}")
+    m = _geometry_model(57, 70, 75, 700, 1e-4, sir=False, sigma=1.0)
+    tt, R = _oracle_of(m).tt.T, _oracle_of(m).R
+    sg = rng(34).standard_normal((B, 75, 700))
+    ref = O.transpose_das(np.transpose(sg, (0, 2, 1)), tt, R)
+    sd = torch.tensor(sg, dtype=torch.float32).cuda()
+    out = {}
+    for v in (55, 56, 57, 58, -1):
+        m.plan.set_launch(B, v, 0)
+        out[v] = m.plan.transpose(sd, model=False).cpu().numpy().reshape(B, -1)
+        assert rel_l2(out[v], ref) < TOL_OP, v
+    assert any(np.array_equal(out[-1], out[v]) for v in (55, 56, 57, 58))
+
+
+@pytest.mark.parametrize("B", [4, 16, 17, 33])
+@pytest.mark.parametrize("h,rows", [(1e-4, 256), (6e-5, 192), (2e-5, 128)])
+def test_sir_transpose_groups_many_detectors(h, rows, B):
+    """The matrix-core SIR transpose with more than eight detectors in a group and a shorter last group (75
+    detectors in groups of 19 and 10), for the three sizes of its row buffer (the samples that a tile's pairs
+    span, three rows each, in steps of 64 rows)."""
+    import torch
+    from mbrec.model import DevicePlan
+    Nz, Nx, D, R, Ls = 37, 53, 75, 2.6666666666666665, 31
+    _log(f"SIR groups 75 detectors B={B} h={h}")
+    tt = geometry_tt(Nz, Nx, h, D, 0.01, 160.0, 1500.0, 4e7).reshape(D, -1)
+    tt = tt - int(tt.min()) + 30
+    nT = int(tt.max()) + 60
+    g = rng(902)
+    nsir = 40
+    se = np.zeros((nsir, 2), dtype=np.int32)
+    for k in range(nsir):
+        se[k, 0] = g.integers(3, 6)
+        se[k, 1] = se[k, 0] + g.integers(14, 25) - 1
+    sir = g.standard_normal((nsir, Ls))
+    sidx = g.integers(1, nsir + 1, size=(D, Nz * Nx)).astype(np.int32)
+    first = np.floor(tt).astype(int).reshape(D, Nx, Nz) + se[sidx - 1, 0].reshape(D, Nx, Nz)
+    last = np.floor(tt).astype(int).reshape(D, Nx, Nz) + se[sidx - 1, 1].reshape(D, Nx, Nz)
+    span = max((last[:, x:x + 16, z:z + 16].max(axis=(1, 2)) - first[:, x:x + 16, z:z + 16].min(axis=(1, 2))).max()
+               for x in range(0, Nx, 16) for z in range(0, Nz, 16)) + 1
+    assert rows - 64 < 3 * span + 1 <= rows or rows == 128 and 3 * span + 1 <= rows
+    plan = DevicePlan(Nz, Nx, D, nT, R, tt, sir=(sidx, sir, se))
+    sg = g.standard_normal((B, D, nT))
+    ref = O.transpose_sir(np.transpose(sg, (0, 2, 1)), sidx.T, np.ascontiguousarray(tt.T), sir.T, se.T, R)
+    sd = torch.tensor(sg, dtype=torch.float32).cuda()
+    for v in (-1, 59, 60, 61, 62):
+        plan.set_launch(B, v, 0)
+        assert rel_l2(plan.transpose(sd, model=False).cpu().numpy().reshape(B, -1), ref) < TOL_OP, v
+
+
 def test_one_sinogram_tile_variants_match_oracle():
     """Every one-sinogram tile form on a real arc geometry (the tile windows fit the LDS only
     for smooth travel times): forward choices 2, 3 (record streaming), 5, 6, 7 (tile form, thread

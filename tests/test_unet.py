@@ -343,3 +343,43 @@ def test_conv3x3_bf16_beyond_32_bit_slots(require_gpu, Cout, relu):
         assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 1e-5)
     del x, y
     torch.cuda.empty_cache()
+
+
+@pytest.mark.gpu
+def test_unet_forward_repeats_itself(require_gpu):
+    """No bit of an image's estimate depends on the call, on the other images of the batch or on its place among
+    them (a sum's order is that of its channels and taps)."""
+    import torch
+    from mbrec.warmstart import UNet
+    net = UNet(32, seed=5)
+    x = torch.as_tensor(rng(41).uniform(0, 1, (5, 40, 72)).astype(np.float32)).cuda()
+    y = net.forward(x).clone()
+    assert torch.equal(net.forward(x), y)
+    for b in (0, 2, 4):
+        assert torch.equal(net.forward(x[b:b + 1].contiguous())[0], y[b])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Cin,Cout", [(38, 32, 32), (19, 256, 256), (38, 384, 128)])
+def test_conv3x3_bf16_is_the_rounded_sum(require_gpu, H, Cin, Cout):
+    """A layer's output is the FP64 sum rounded to bfloat16 but for values within the FP32 sum's error of a tie:
+    2^-24 of the sum of magnitudes per product, 9 Cin products, and such a value is off by one step."""
+    import torch
+    from mbrec import _lib
+    g = rng(42)
+    x = _bf16_tensor(np.maximum(g.standard_normal((2, H, H, Cin)), 0))
+    w = _bf16_tensor(g.standard_normal((Cout, 3, 3, Cin)) / np.sqrt(9 * Cin))
+    xd, wd = x.cuda(), w.cuda()
+    yd = torch.empty((2, H, H, Cout), dtype=torch.bfloat16, device="cuda")
+    _lib.check(_lib.lib().mbrec_conv3x3_bf16(xd.data_ptr(), wd.data_ptr(), None, yd.data_ptr(), 2, H, H, Cin, Cout, 0,
+                                             _lib.stream_handle()))
+
+    def conv(a, b):
+        return torch.nn.functional.conv2d(a.permute(0, 3, 1, 2), b.permute(0, 3, 1, 2), padding=1).permute(0, 2, 3, 1)
+    want, mag = conv(x.double(), w.double()), conv(x.double().abs(), w.double().abs())
+    got = yd.cpu()
+    err = 9 * Cin * 2.0 ** -24 * mag
+    lo, hi = (want - err).float().bfloat16().float(), (want + err).float().bfloat16().float()
+    assert ((got.float() >= lo) & (got.float() <= hi)).all()
+    # observed 2e-4 at most (direct kernels with another order of the sums: the same)
+    assert (got != want.float().bfloat16()).float().mean() < 1e-3
