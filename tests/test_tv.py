@@ -280,7 +280,8 @@ def test_tv_scratch_is_given_back(require_gpu):
         SB_ITV2(g, mu)
         torch.cuda.empty_cache()
         kept = free - torch.cuda.mem_get_info()[0]
-        assert 7 * 16 * 160000 * 8 <= kept <= (1 << 30) + (64 << 20)
+        # 143 MB of arrays; other small allocations of the process come and go with their granularity (2 MB)
+        assert 7 * 16 * 160000 * 8 - (16 << 20) <= kept <= (1 << 30) + (64 << 20)
         mbrec.release_scratch() if release == "call" else plan.close()
         plan.close()
         assert free - torch.cuda.mem_get_info()[0] < 32 << 20
