@@ -112,11 +112,8 @@ hipError_t device_malloc(void **p, size_t bytes)
     return hipMalloc(p, bytes);
 }
 
-static void ensure_sir_groups(Plan *p);
-
 int ensure_work(Plan *p, int B)
 {
-    if (p->use_sir && batch_stride(B) >= 4) ensure_sir_groups(p);
     const size_t need_h = std::max<size_t>((size_t)p->D * p->nbk * p->WL, 1);
     if (B <= p->bcap && p->d_hpart && p->work_bytes && need_h * batch_stride(p->bcap) * sizeof(float) <=
                                                              p->work_bytes)
@@ -558,8 +555,8 @@ static int build_sir_tiles(Plan *p, const std::vector<int32_t> &slot_pix, const 
 // the range check is the window's (a pair's offset points at its weight on the window's first
 // sample: the zero margins of d_sirw give the rest).  No tables where a (tile, detector) needs more
 // than 24 groups or 256 rows, or the axis is shorter than a window.
-// Built at a plan's first batch (3.5 KB per (tile, detector): 0.57 GB at 400^2 x 256, and as much on the
-// host meanwhile), from the plan's own tables; where memory runs out the other SIR forms run.
+// 3.5 KB per (tile, detector): 0.57 GB at 400^2 x 256, and as much on the host meanwhile; where memory
+// runs out the plan does without, and the other SIR forms run.
 static void free_sir_groups(Plan *p)
 {
     for (void *q : {(void *)p->d_sghdr, (void *)p->d_sgent, (void *)p->d_sgslot})
@@ -570,20 +567,14 @@ static void free_sir_groups(Plan *p)
     p->d_sgent = nullptr;
     p->d_sgslot = nullptr;
     p->sg_rows = 0;
-    p->sg_tried = false;
 }
 
-static int build_sir_groups(Plan *p)
+static int build_sir_groups(Plan *p, const std::vector<int32_t> &slot_pix, const std::vector<int32_t> &tq,
+                            const int32_t *sidx, const int32_t *win, int Ls, int maxlen)
 {
     const BinGeom &g = p->geom;
-    const int span = g.nT + 2 * g.K, half = p->Ls / 2, ntile = p->Pd / 256;
-    const int maxlen = p->sir_maxlen;
+    const int span = g.nT + 2 * g.K, half = Ls / 2, ntile = p->Pd / 256;
     if (!p->d_sirw || maxlen > kSgWin || span < kSgWin) return MBREC_OK;
-    std::vector<int32_t> slot_pix(p->Pd), tq((size_t)p->D * p->Pd), sidx(tq.size()), win(2 * (size_t)p->Nsir);
-    MBREC_HIP(hipMemcpy(slot_pix.data(), p->d_pix, sizeof(int32_t) * slot_pix.size(), hipMemcpyDeviceToHost));
-    MBREC_HIP(hipMemcpy(tq.data(), p->d_tq, sizeof(int32_t) * tq.size(), hipMemcpyDeviceToHost));
-    MBREC_HIP(hipMemcpy(sidx.data(), p->d_sidx, sizeof(int32_t) * sidx.size(), hipMemcpyDeviceToHost));
-    MBREC_HIP(hipMemcpy(win.data(), p->d_swin, sizeof(int32_t) * win.size(), hipMemcpyDeviceToHost));
     const int stride = maxlen + 2 * kSirWinPad;
     const size_t ntd = (size_t)ntile * p->D;
     // zeroed tile by tile by the threads below
@@ -666,19 +657,18 @@ static int build_sir_groups(Plan *p)
     return MBREC_OK;
 }
 
-static void ensure_sir_groups(Plan *p)
+static void try_sir_groups(Plan *p, const std::vector<int32_t> &slot_pix, const std::vector<int32_t> &tq,
+                           const int32_t *sidx, const int32_t *win, int Ls, int maxlen)
 {
-    if (p->sg_tried) return;
     bool ok = false;
     try {
-        ok = build_sir_groups(p) == MBREC_OK;
+        ok = build_sir_groups(p, slot_pix, tq, sidx, win, Ls, maxlen) == MBREC_OK;
     } catch (const std::exception &) {   // no host memory
     }
     if (!ok) {
         p->table_bytes += p->sg_bytes;   // counted as the finished tables are
         free_sir_groups(p);
     }
-    p->sg_tried = true;
 }
 
 int build_records(Plan *p, const std::vector<int32_t> &slot_pix, const std::vector<int32_t> &tq,
@@ -1120,6 +1110,7 @@ int mbrec_plan_set_sir(mbrec_plan h, const int32_t *sirIdx, const double *sir, i
         p->Nsir_build = Nsir;
         if ((rc = build_sir_pull(p, slot_pix, tq, sidx.data(), win.data(), Ls, sirf.data()))) return rc;
         if ((rc = build_sir_tiles(p, slot_pix, tq, sidx.data(), win.data(), Ls))) return rc;
+        try_sir_groups(p, slot_pix, tq, sidx.data(), win.data(), Ls, maxlen);
     }
     p->use_sir = 1;
     p->Ls = Ls;

@@ -138,7 +138,6 @@ struct Plan {
     int2 *d_sgent = nullptr;
     uint32_t *d_sgslot = nullptr;
     int sg_rows = 0;             // staged bin rows: 64 * ceil(longest / 64)
-    bool sg_tried = false;       // the tables have been built, or found not to fit
     size_t sg_bytes = 0;
     int32_t *d_srec_off = nullptr;
     int sp_lo = 0, sp_n = 0, Nsir_build = 0;

@@ -298,29 +298,39 @@ def test_sir_transpose_groups_match_oracle(B, crop):
     assert ran == 4      # the geometry's pairs fit the groups
 
 
-def test_sir_group_tables_come_with_the_first_batch():
-    """The tables of the matrix-core SIR transpose (3.5 KB per 256-pixel tile and detector) are built for the
-    first batch: a plan used for one sinogram does without.  New SIR tables rebuild them."""
+def test_sir_group_tables_follow_the_sir_tables():
+    """The tables of the matrix-core SIR transpose go with SIR windows too long for them (36 taps; the older forms
+    run) and come back with the first ones, and the transpose that allocates nothing finds them there."""
     import torch
+    from mbrec import _lib
     _log("SIR group tables")
-    D, nT = 64, 1000
-    m = _geometry_model(200, 200, D, nT, 1e-4, sir=True, sigma=1.0)
-    groups = 13 * 13 * D * 3584
-    sg = torch.tensor(rng(39).standard_normal((4, D, nT)), dtype=torch.float32).cuda()
-    torch.cuda.synchronize()
-
-    def used(B):
-        before = torch.cuda.mem_get_info()[0]
-        m.plan.transpose(sg[:B].contiguous(), model=False)
-        torch.cuda.synchronize()
-        return before - torch.cuda.mem_get_info()[0]
-    assert used(1) < groups
-    assert used(4) > groups
-    x = m.plan.transpose(sg, model=False).cpu().numpy()
-    d = m.Data
-    m.plan.set_sir(d.SPMRIndices.reshape(D, -1), d.SPMR, d.SPMRTimestepIndexStartAndEnd)
-    m.plan.set_launch(4, 61, 0)
-    assert np.array_equal(m.plan.transpose(sg, model=False).cpu().numpy(), x)
+    D, nT, Nz, Nx = 12, 300, 40, 44
+    m = _geometry_model(Nz, Nx, D, nT, 1e-4, sir=True, sigma=1.0)
+    d, plan = m.Data, m.plan
+    tt, R = _oracle_of(m).tt.T, _oracle_of(m).R
+    first = (d.SPMRIndices.reshape(D, -1), d.SPMR, d.SPMRTimestepIndexStartAndEnd)
+    g = rng(39)
+    long_ = (g.integers(1, 6, size=(D, Nz * Nx)).astype(np.int32), g.standard_normal((5, 61)),
+             np.tile(np.array([[12, 47]], dtype=np.int32), (5, 1)))
+    sg = g.standard_normal((4, D, nT))
+    sd = torch.tensor(sg, dtype=torch.float32).cuda()
+    seen = []
+    for sidx, table, se in (first, long_, first):
+        plan.set_sir(sidx, table, se)
+        if se is long_[2]:
+            with pytest.raises(Exception):
+                plan.set_launch(4, 61, 0)
+        else:
+            got = torch.full((4, Nz * Nx), float("nan"), device="cuda")
+            _lib.check(_lib.lib().mbrec_model_transpose_noalloc_dev(plan.h, sd.data_ptr(), got.data_ptr(), 4,
+                                                                    _lib.stream_handle()))
+            assert torch.equal(got, plan.transpose(sd).reshape(4, -1))
+            plan.set_launch(4, 61, 0)
+        ref = O.transpose_sir(np.transpose(sg, (0, 2, 1)), sidx.T, tt, table.T, se.T, R)
+        seen.append(plan.transpose(sd, model=False).cpu().numpy().reshape(4, -1))
+        assert rel_l2(seen[-1], ref) < TOL_OP
+    assert np.array_equal(seen[0], seen[2])
+    assert 0 < plan.device_bytes < 1 << 40
 
 
 @pytest.mark.parametrize("sir", [False, True])
