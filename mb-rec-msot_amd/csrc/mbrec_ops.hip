@@ -4491,7 +4491,8 @@ static int default_gather_variant(const Plan *p, int Bp)
         // per CU, in two detector groups, four where those leave CUs without one.  Measured, stage time
         // against the former choices: 301 x 333 x 28 0.30 / 1.22 ms (the 64-sinogram form 0.60), x 13
         // 0.19 / 0.57 ms, x 9 0.18 / 0.43 ms (x 8: 0.17 / 0.13, so Bp = 8 stays), 400^2 x 64
-        // 0.78 / 0.84 ms (x 100: 2.4 / 1.7, so larger batches stay).
+        // 0.78 / 0.84 ms.  Larger batches stay with the 64-wide form (400^2 x 65 1.57 / 1.77 ms, x 72 1.57 /
+        // 1.61, x 100 1.7 / 2.4), though three chunks of 32 would be faster for 77 to 96 (x 96 1.61 / 1.16).
         const bool small = Bp <= 16;
         const int tiles = p->Pd / 256, chunks = small ? 1 : (Bp + 31) / 32;
         const bool few = tiles * chunks * 2 < (small ? 1024 : 512);
